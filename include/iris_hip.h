@@ -181,7 +181,8 @@ int iris_gemm_bf16(const void* a, const void* b, const float* bias, void* c, int
  * with direct-to-LDS refills, the SiLU epilogue's; 11 and 12 the four-wave 32x32x16 kernel at
  * 256x256 and 192x256; 13-17 the four-wave 16x16x32 kernel at 288x160, 256x160, 128x160,
  * 256x256 and 192x256, the automatic choice for plain, bias and SwiGLU outputs) or restore the
- * automatic choice (-1). A forced tile of the other MFMA shape rounds differently from the
+ * automatic choice (-1); 18-26 small tiles, 32x64 to 192x128, of the ring kernel, which need
+ * k >= 64 x the K tiles of their ring). A forced tile of the other MFMA shape rounds differently from the
  * automatic one. The setting is per thread. No counterpart in the reference. */
 int iris_gemm_force_tile(int tile);
 

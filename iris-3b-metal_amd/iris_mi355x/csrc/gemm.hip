@@ -7,14 +7,16 @@
 // free, and workgroup ids are remapped so that the tiles running concurrently on one XCD form
 // an 8 x 4 block and share their operands through that XCD's L2.
 //
-// Three kernels:
+// Four kernels:
 // - gemm_w4h_kernel (the default for plain, bias and SwiGLU outputs and the q|k|v store): four
 //   waves, one per SIMD, in a 2 x 2 grid of v_mfma_f32_16x16x32_bf16 blocks; K tiles staged
 //   through registers (16-byte buffer loads two K tiles ahead) into a 2-stage LDS ring;
 //   288 x 160, 256 x 160, 128 x 160, 256 x 256 and 192 x 256 tiles. gemm_w4h_pair_kernel runs
 //   two of its GEMMs in one grid (SwiGLU's two column parts; the q|k|v store and the gate
 //   columns beside it), which saves the boundary between two launches.
-// - gemm_w4_kernel: the same design on v_mfma_f32_32x32x16_bf16 (256 x 256, 192 x 256),
+// - gemm_ring_kernel (few rows): four waves on the same MFMA, small tiles (32 x 64 .. 192 x 128) with
+//   K tiles global -> LDS by buffer_load_dwordx4 ... lds, three to eight of them in flight.
+// - gemm_w4_kernel: gemm_w4h_kernel's design on v_mfma_f32_32x32x16_bf16 (256 x 256, 192 x 256),
 //   forced-only (a tuning and test reference).
 // - gemm_kernel: eight waves, K tiles global -> LDS with buffer_load_dwordx4 ... lds into a ring
 //   of STAGES buffers (no register staging; a 32-bit VGPR byte offset per load, the K position
@@ -263,6 +265,73 @@ __device__ __forceinline__ void qk_store(bf16* cl, const TileJob& job, int N, lo
                      : qk.k + ((static_cast<long>(b) * qk.kv_heads + head) * qk.n_dst + pos) * 128;
     *reinterpret_cast<bf16x8*>(dst + 8 * (c & 15)) = v;
   }
+}
+
+// kEpiQkRope on 128-wide tiles (one head, or 128 plain columns, per tile), once the BF16 tile is
+// staged in LDS (16-byte chunk c of row r at c ^ (r & 15)): 16 lanes per row, one chunk each, so a
+// head is normed and rotated by head_norm_rope in registers and leaves as whole 256-byte rows; the
+// V heads transposed per 16-position group (rows_per_batch and dst_offset are multiples of 16 with
+// vt, so a group lies inside one batch item); the other columns to C.
+template <int BM, int NW>
+__device__ __forceinline__ void qk_store_head(const bf16* cl, const TileJob& job, long ldc, const QkRope& qk) {
+  constexpr int OUT_N = 128;
+  const int tid = threadIdx.x;
+  const int M = job.m, m0 = job.tm * BM, n0 = job.tn * OUT_N;
+  const int nq = qk.heads * 128, nqk = nq + qk.kv_heads * 128, nqkv = nqk + qk.kv_heads * 128;
+  const int rpb = job.group ? qk.rows_per_batch1 : qk.rows_per_batch0;
+  const int dst_offset = job.group ? qk.dst_offset1 : qk.dst_offset0;
+  const int c = tid & 15;
+  auto chunk = [&](int r) { return *reinterpret_cast<const bf16x8*>(cl + r * OUT_N + 8 * (c ^ (r & 15))); };
+  if (n0 < nqk) {
+    const bool is_q = n0 < nq;
+    const int head = (is_q ? n0 : n0 - nq) >> 7;
+    const int heads = is_q ? qk.heads : qk.kv_heads;
+    bf16* dst = is_q ? qk.q : qk.k;
+    const float* gains = is_q ? (job.group ? qk.q_weight1 : qk.q_weight0) : (job.group ? qk.k_weight1 : qk.k_weight0);
+    float wg[8];
+    load8(gains + 8 * c, wg);
+#pragma unroll 2
+    for (int r = tid >> 4; r < BM; r += 4 * NW) {
+      const int m = min(m0 + r, M - 1);  // (a row past M normalises zeros or stale values, not stored)
+      const int b = m / rpb;
+      const long pos = dst_offset + (m - b * rpb);
+      const f32x4 cs = load4(qk.cos + pos * 64 + 4 * c);
+      const f32x4 sn = load4(qk.sin + pos * 64 + 4 * c);
+      const bf16x8 v = chunk(r);
+      float a[8], y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] = to_f32(v[e]);
+      head_norm_rope(a, wg, cs, sn, qk.eps, y);
+      if (m0 + r < M) store8(dst + ((static_cast<long>(b) * heads + head) * qk.n_dst + pos) * 128 + 8 * c, y);
+    }
+    return;
+  }
+  if (qk.vt && n0 < nqkv) {
+    // thread t gathers dim t % 128 for the 8 positions 8 c8 .. 8 c8 + 7 (slot order of vt_slot)
+    const int d = tid & 127;
+    const int vh = (n0 - nqk) >> 7;
+#pragma unroll 2
+    for (int c8 = tid >> 7; c8 < BM / 8; c8 += NW / 2) {  // (wave-uniform)
+      const int g0 = 16 * (c8 >> 1);                      // the 16-position group's first tile row
+      if (m0 + g0 >= M) continue;
+      const int b = (m0 + g0) / rpb;
+      const long p0 = dst_offset + (m0 + g0 - b * rpb) + 8 * (c8 & 1);
+      bf16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int i = g0 + vt_slot(8 * (c8 & 1) + e);
+        o[e] = cl[i * OUT_N + 8 * ((d >> 3) ^ (i & 15)) + (d & 7)];
+      }
+      *reinterpret_cast<bf16x8*>(qk.vt + ((static_cast<long>(b) * qk.kv_heads + vh) * 128 + d) * static_cast<long>(qk.n_vt) +
+                                 p0) = o;
+    }
+    return;
+  }
+  bf16* __restrict__ C = static_cast<bf16*>(job.c);
+#pragma unroll 4
+  for (int r = tid >> 4; r < BM; r += 4 * NW)
+    if (m0 + r < M)
+      __builtin_nontemporal_store(chunk(r), reinterpret_cast<bf16x8*>(C + static_cast<long>(m0 + r) * ldc + n0 + 8 * c));
 }
 
 // Epilogue shared by the kernels: acc[i][j][r] = C[m, n] with n = tile + wave col + 32 i +
@@ -855,10 +924,12 @@ __device__ __forceinline__ void store_tile16(f32x4 (&acc)[FN][FM], bf16* lds, co
     static_assert(BM * PITCH <= RING, "output tile must fit in the LDS ring");
     bf16* cl = lds;
     __syncthreads();
-    __shared__ float qk_gain[EPI == kEpiQkRope ? 256 : 1];
-    [[maybe_unused]] f32x4 qk_cos[EPI == kEpiQkRope ? 16 : 1], qk_sin[EPI == kEpiQkRope ? 16 : 1];
-    if constexpr (EPI == kEpiQkRope) {
-      static_assert(BM == 64 * NW && BN == 256 && SWZ, "one 256-wide tile row per thread");
+    constexpr bool QK2 = EPI == kEpiQkRope && BN == 256;  // two heads per row, one row per thread
+    static_assert(EPI != kEpiQkRope || QK2 || BN == 128, "one or two whole heads per tile row");
+    __shared__ float qk_gain[QK2 ? 256 : 1];
+    [[maybe_unused]] f32x4 qk_cos[QK2 ? 16 : 1], qk_sin[QK2 ? 16 : 1];
+    if constexpr (QK2) {
+      static_assert(BM == 64 * NW && SWZ, "one 256-wide tile row per thread");
       qk_tables<BM>(job, qk, qk_gain, qk_cos, qk_sin);
     }
 #pragma unroll
@@ -877,8 +948,11 @@ __device__ __forceinline__ void store_tile16(f32x4 (&acc)[FN][FM], bf16* lds, co
     }
     __syncthreads();
     mid();
-    if constexpr (EPI == kEpiQkRope) {
+    if constexpr (QK2) {
       qk_store<BM, NW>(cl, job, N, ldc, qk, qk_gain, qk_cos, qk_sin);
+      return;
+    } else if constexpr (EPI == kEpiQkRope) {
+      qk_store_head<BM, NW>(cl, job, ldc, qk);
       return;
     }
     constexpr int CHUNKS = OUT_N / 8;
@@ -1197,6 +1271,184 @@ __global__ __launch_bounds__(256) void gemm_w4h_pair_kernel(GemmArgs p1, GemmArg
   }
 }
 
+// The small-tile GEMM of the 16 x 16 x 32 family: four waves in a 2 x 2 grid over a BM x BN tile,
+// K tiles of 64 fetched by `buffer_load_dwordx4 ... lds` into a ring of STAGES buffers.
+//
+// What bounds it: with few rows a launch is a stream of weights, and a CU takes ~55 bytes a clock of
+// it into LDS (128 x 128, 107 K tiles: 31 us for the loads alone, 29 for the MFMAs alone, 50 to 57
+// for all), so small tiles that put the call on every CU are worth their extra traffic. A weight
+// read from HBM takes ~2000 clocks, a K tile 128 .. 512 of MFMAs: the ring keeps STAGES - 1 K
+// tiles (72 .. 140 KB per CU) in flight with no registers, where the register-staged kernels
+// above hold two. Measured (2560 columns, K = 6848, weights from HBM): 333 rows 62 -> 24 us, 64
+// rows 59 -> 22 us, 924 rows 62 -> 49 us; SwiGLU 333 x 13696 x 2560 45 -> 34 us; q|k|v|gate of a
+// 256 x 256 image with 77 text tokens 109 -> 24 us. Each output sums k in the order of
+// gemm_w4h_kernel on the same MFMA with the operands in the same roles, so the results are equal
+// bit for bit.
+//
+// One barrier per K tile: the fragments of tile t + 1 are read from LDS into the second register
+// buffer while tile t is multiplied from the first. The wait before that barrier has tile t + 1
+// landed (STAGES - 2 tiles may still fly) and this wave's reads of tile t done, so behind the
+// barrier stage t % STAGES is refilled with tile t + STAGES. The last STAGES tiles issue no loads.
+// The loads follow the reads: a load issued into a full address queue holds up the MFMAs and
+// reads behind it. The MFMAs are builtins here (the accumulators are few; the in-place assembly
+// of gemm_w4h_kernel pads hazards only at the edges of a run, and with AGPRs to spare the compiler
+// copies accumulators inside it). Measured level and dropped: fragments two tiles ahead; loads
+// dealt between the MFMAs.
+template <int BM, int BN, int STAGES>
+constexpr unsigned ring_lds_bytes() {
+  return static_cast<unsigned>(STAGES) * (BM + BN) * 64u * sizeof(bf16);
+}
+
+template <int BM, int BN, int STAGES, int EPI, typename TC>
+__global__ __launch_bounds__(256) void gemm_ring_kernel(GemmArgs p) {
+  constexpr int BK = 64, NW = 4;
+  constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
+  constexpr int CPR = BK / 8, RPL = 64 / CPR;  // 16-byte chunks per row, rows per 1 KB wave load
+  constexpr int A_LOADS = BM / RPL / NW, B_LOADS = BN / RPL / NW, LPW = A_LOADS + B_LOADS;
+  constexpr int NR = 2 * (FN + FM), NM = 2 * FN * FM;  // fragment reads and MFMAs per K tile
+  constexpr int A_STAGE = BM * BK, STAGE = (BM + BN) * BK;
+  static_assert(WM % 16 == 0 && WN % 16 == 0 && A_LOADS * RPL * NW == BM && B_LOADS * RPL * NW == BN,
+                "tile / wave split");
+  static_assert(STAGES >= 3 && (STAGES - 1) * LPW < 64, "loads in flight fit vmcnt");
+  static_assert(STAGES * STAGE * sizeof(bf16) == ring_lds_bytes<BM, BN, STAGES>(), "LDS ring");
+  extern __shared__ __attribute__((aligned(1024))) bf16 lds[];  // ring_lds_bytes at launch
+
+  const TileJob job = locate_tile<BM, BN>(p);
+  const int N = p.n;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int l16 = lane & 15;
+  const int q4 = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: LDS targets stay scalar
+  const int wm = w >> 1, wn = w & 1;
+
+  // addresses as in gemm_w4h_tiles: lane l of load j fetches the chunk that belongs at byte 16 l of
+  // that 1 KB block; rows past an operand's end read zeros (or, past 2^32 bytes, wrap inside the
+  // buffer) and reach only outputs that are not stored
+  const int ld_r = lane / CPR;
+  const int ld_p = lane % CPR;
+  const unsigned lda2 = 2u * static_cast<unsigned>(p.lda), ldb2 = 2u * static_cast<unsigned>(p.ldb);
+  unsigned voff[2][2];  // [operand][parity of the load]
+#pragma unroll
+  for (int op = 0; op < 2; ++op)
+#pragma unroll
+    for (int par = 0; par < 2; ++par) {
+      const int r = (w * (op ? B_LOADS : A_LOADS) + par) * RPL + ld_r;
+      const unsigned row = static_cast<unsigned>((op ? job.tn * BN : job.tm * BM) + r);
+      voff[op][par] = row * (op ? ldb2 : lda2) + 16u * static_cast<unsigned>(ld_p ^ swz<BK>(r));
+    }
+  const __amdgpu_buffer_rsrc_t rsrc_a =
+      __builtin_amdgcn_make_buffer_rsrc((void*)job.a, (short)0, job.m * static_cast<int>(p.lda) * 2, kBufferFlags);
+  const __amdgpu_buffer_rsrc_t rsrc_b =
+      __builtin_amdgcn_make_buffer_rsrc((void*)job.b, (short)0, N * static_cast<int>(p.ldb) * 2, kBufferFlags);
+  auto load1 = [&](int kt, int stage, int i) {  // load i of K tile kt: the weight's, then the activation's
+    const int op = i < B_LOADS ? 1 : 0;
+    const int j = op ? i : i - B_LOADS;
+    buffer_load_lds16(op ? rsrc_b : rsrc_a,
+                      lds + stage * STAGE + (op ? A_STAGE + (w * B_LOADS + j) * RPL * BK : (w * A_LOADS + j) * RPL * BK),
+                      static_cast<int>(voff[op][j & 1]),
+                      static_cast<int>(static_cast<unsigned>(kt * BK * 2) +
+                                       static_cast<unsigned>((j & ~1) * RPL) * (op ? ldb2 : lda2)));
+  };
+
+  int frag_off[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) frag_off[ks] = l16 * BK + 8 * ((4 * ks + q4) ^ swz<BK>(l16));
+  bf16x8 wf[2][2][FN], xf[2][2][FM];  // [buffer][k-step]
+  auto read1 = [&](int stage, int buf, int i) {  // fragment i of a K tile: k-step 0's, then k-step 1's
+    const int ks = i / (FN + FM), f = i % (FN + FM);
+    const bf16* s = lds + stage * STAGE + frag_off[ks];
+    if (f < FN)
+      wf[buf][ks][f] = *reinterpret_cast<const bf16x8*>(s + A_STAGE + (wn * WN + 16 * f) * BK);
+    else
+      xf[buf][ks][f - FN] = *reinterpret_cast<const bf16x8*>(s + (wm * WM + 16 * (f - FN)) * BK);
+  };
+  f32x4 acc[FN][FM];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{};
+  // (the empty asm keeps the compiler's own memory operations on their side of the barrier)
+  auto publish = [&](auto pending_) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    wait_vmcnt_lgkm0<decltype(pending_)::value * LPW>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using Z = std::integral_constant<int, 0>;
+
+  const int KT = p.k / BK;  // >= STAGES (the launch sees to it)
+#pragma unroll
+  for (int t = 0; t < STAGES; ++t)
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) load1(t, t, i);
+  publish(std::integral_constant<int, STAGES - 1>{});  // tile 0 has landed
+#pragma unroll
+  for (int i = 0; i < NR; ++i) read1(0, 0, i);
+  int stage = 0, t = 0;  // tile t sits in stage `stage`
+  // multiply tile t from buffer `buf`. READS: tile t + 1 exists: it is waited for (`pending` later
+  // tiles may be in flight) and its fragments are read into the other buffer; LOADS: tile
+  // t + STAGES exists and is fetched
+  auto step = [&](auto buf_, auto loads_, auto reads_, auto pending_) {
+    constexpr int buf = decltype(buf_)::value;
+    constexpr bool LOADS = decltype(loads_)::value != 0, READS = decltype(reads_)::value != 0;
+    const int next = stage + 1 == STAGES ? 0 : stage + 1;
+    if constexpr (READS) {
+      publish(pending_);
+#pragma unroll
+      for (int i = 0; i < NR; ++i) read1(next, buf ^ 1, i);
+    }
+    if constexpr (LOADS) {
+#pragma unroll
+      for (int i = 0; i < LPW; ++i) load1(t + STAGES, stage, i);
+    }
+#pragma unroll
+    for (int idx = 0; idx < NM; ++idx) {
+      const int ks = idx / (FN * FM), i = idx % (FN * FM) / FM, j = idx % FM;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[buf][ks][i], xf[buf][ks][j], acc[i][j], 0, 0, 0);
+    }
+    // order: the reads behind the first MFMAs, then the loads, then the remaining MFMAs
+    if constexpr (READS) {
+      constexpr int DENSE = (NR + NM - 1) / NM;  // reads per MFMA
+#pragma unroll
+      for (int i = 0; i < (NR + DENSE - 1) / DENSE; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, DENSE, 0);  // DS read
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // MFMA
+      }
+      if constexpr (LOADS) __builtin_amdgcn_sched_group_barrier(0x010, LPW, 0);  // VMEM
+      __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+    }
+    stage = next;
+    ++t;
+  };
+  using O = std::integral_constant<int, 1>;
+  auto main_step = [&](auto buf_) { step(buf_, O{}, O{}, std::integral_constant<int, STAGES - 2>{}); };
+  // the last STAGES tiles, `left` of them still to do, the first in fragment buffer `buf`
+  auto tail = [&](auto self, auto left_, auto buf_) -> void {
+    constexpr int left = decltype(left_)::value, buf = decltype(buf_)::value;
+    if constexpr (left > 1) {
+      step(buf_, Z{}, O{}, std::integral_constant<int, left - 2>{});
+      self(self, std::integral_constant<int, left - 1>{}, std::integral_constant<int, buf ^ 1>{});
+    } else {
+      step(buf_, Z{}, Z{}, Z{});
+    }
+  };
+  const int mains = KT - STAGES;
+  for (int i = mains / 2; i > 0; --i) {
+    main_step(Z{});
+    main_step(O{});
+  }
+  if (mains % 2) {
+    main_step(Z{});
+    tail(tail, std::integral_constant<int, STAGES>{}, O{});
+  } else {
+    tail(tail, std::integral_constant<int, STAGES>{}, Z{});
+  }
+  store_tile16<BM, BN, WM, WN, FM, FN, NW, STAGES * STAGE, EPI, TC>(acc, lds, job, N, p.ldc, wm, wn, p.qk, [] {});
+}
+
 template <int BM, int BN, int BK, int STAGES, int WGM, int WGN, int PARTS>
 int launch_tile(GemmArgs& args, int c_dtype, int epilogue, hipStream_t stream) {
   const dim3 grid(args.total_tiles);
@@ -1289,11 +1541,43 @@ int launch_w4h(GemmArgs& args, int c_dtype, int epilogue, hipStream_t stream) {
   return check_launch("gemm_bf16");
 }
 
+template <int BM, int BN, int STAGES>
+int launch_ring(GemmArgs& args, int c_dtype, int epilogue, hipStream_t stream) {
+  if (args.k / kBK < STAGES) return fail(IRIS_E_UNSUPPORTED, "gemm: the %dx%d ring needs k >= %d", BM, BN, STAGES * kBK);
+  const dim3 all(args.total_tiles);
+  constexpr unsigned lds = ring_lds_bytes<BM, BN, STAGES>();
+  if (epilogue == IRIS_EPI_NONE) {
+    if (c_dtype == IRIS_BF16)
+      gemm_ring_kernel<BM, BN, STAGES, IRIS_EPI_NONE, bf16><<<all, 256, lds, stream>>>(args);
+    else
+      gemm_ring_kernel<BM, BN, STAGES, IRIS_EPI_NONE, float><<<all, 256, lds, stream>>>(args);
+    return check_launch("gemm_bf16");
+  }
+  if (epilogue == IRIS_EPI_SILU_MUL) {
+    if constexpr (BN / 2 % 64 == 0) {
+      if (c_dtype == IRIS_BF16)
+        gemm_ring_kernel<BM, BN, STAGES, IRIS_EPI_SILU_MUL, bf16><<<all, 256, lds, stream>>>(args);
+      else
+        gemm_ring_kernel<BM, BN, STAGES, IRIS_EPI_SILU_MUL, float><<<all, 256, lds, stream>>>(args);
+      return check_launch("gemm_bf16");
+    }
+  }
+  if (epilogue == kEpiQkRope) {
+    if constexpr (BN == 128) {
+      gemm_ring_kernel<BM, BN, STAGES, kEpiQkRope, bf16><<<all, 256, lds, stream>>>(args);
+      return check_launch("gemm_bf16");
+    }
+  }
+  return fail(IRIS_E_UNSUPPORTED, "gemm: the %dx%d ring tile has no such epilogue", BM, BN);
+}
+
 struct TileShape {
   int bm, bn, bk, stages, wgm, wgn, parts;
   bool w4 = false;   // gemm_w4_kernel: four waves of 128 x 128, register-staged refills
   bool w4h = false;  // gemm_w4h_kernel: four waves on the 16 x 16 x 32 MFMA
-  bool swiglu() const { return w4h ? (bn / 2) % 64 == 0 : (bn / wgn / 32) % 2 == 0; }
+  bool ring = false;  // gemm_ring_kernel: the same MFMA, `stages` K tiles in flight
+  bool mfma16() const { return w4h || ring; }
+  bool swiglu() const { return mfma16() ? (bn / 2) % 64 == 0 : (bn / wgn / 32) % 2 == 0; }
 };
 // BM x BN output tile, BK-deep K tiles in a ring of `stages`, wgm x wgn waves, the refill of a
 // K tile spread over `parts` k-steps.
@@ -1316,6 +1600,15 @@ constexpr TileShape kTiles[] = {
     {128, 160, 64, 2, 2, 2, 1, false, true},  // 15: gemm_w4h_kernel, 64 x 80 per wave
     {256, 256, 64, 2, 2, 2, 1, false, true},  // 16: gemm_w4h_kernel, 128 x 128 per wave
     {192, 256, 64, 2, 2, 2, 1, false, true},  // 17: gemm_w4h_kernel, 96 x 128 per wave
+    {32, 64, 64, 8, 2, 2, 1, false, false, true},    // 18: gemm_ring_kernel
+    {64, 64, 64, 8, 2, 2, 1, false, false, true},    // 19: gemm_ring_kernel
+    {96, 64, 64, 7, 2, 2, 1, false, false, true},    // 20: gemm_ring_kernel
+    {128, 64, 64, 6, 2, 2, 1, false, false, true},   // 21: gemm_ring_kernel
+    {32, 128, 64, 7, 2, 2, 1, false, false, true},   // 22: gemm_ring_kernel
+    {64, 128, 64, 6, 2, 2, 1, false, false, true},   // 23: gemm_ring_kernel
+    {96, 128, 64, 5, 2, 2, 1, false, false, true},   // 24: gemm_ring_kernel
+    {128, 128, 64, 4, 2, 2, 1, false, false, true},  // 25: gemm_ring_kernel
+    {192, 128, 64, 3, 2, 2, 1, false, false, true},  // 26: gemm_ring_kernel
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
@@ -1328,6 +1621,9 @@ int launch_index(GemmArgs& args, int c_dtype, int epilogue, hipStream_t stream) 
   } else if constexpr (t.w4h) {
     static_assert(t.bk == 64, "gemm_w4h_kernel tile");
     return launch_w4h<t.bm, t.bn>(args, c_dtype, epilogue, stream);
+  } else if constexpr (t.ring) {
+    static_assert(t.bk == 64, "gemm_ring_kernel tile");
+    return launch_ring<t.bm, t.bn, t.stages>(args, c_dtype, epilogue, stream);
   } else {
     return launch_tile<t.bm, t.bn, t.bk, t.stages, t.wgm, t.wgn, t.parts>(args, c_dtype, epilogue, stream);
   }
@@ -1378,7 +1674,7 @@ bool mfma16_family(int epilogue) { return epilogue == IRIS_EPI_NONE || epilogue 
 
 bool allowed(const Candidate& c, int epilogue) {
   const TileShape t = kTiles[c.tile];
-  return t.w4h == mfma16_family(epilogue) && !(epilogue == IRIS_EPI_SILU_MUL && !t.swiglu()) &&
+  return t.mfma16() == mfma16_family(epilogue) && !(epilogue == IRIS_EPI_SILU_MUL && !t.swiglu()) &&
          !(epilogue == IRIS_EPI_SILU && (t.w4 || t.w4h));
 }
 
@@ -1427,6 +1723,59 @@ SplitPlan plan_split(const int* m, int groups, int n, int epilogue, int forced) 
     if (cost <= best) best = cost, plan.n1 = n1, plan.tile1 = sq.tile, plan.tile2 = t2;
   }
   return plan;
+}
+
+// The ring tiles (gemm_ring_kernel) against the tiles above. Their time is that of the K loop plus
+// what a round costs besides (its first K tiles' latency from HBM, the output), so it depends on K,
+// and they are compared as times: rounds x (K tiles x ktile_us + fixed_us), both measured on one
+// box over 40 and 107 K tiles (2560 columns, K = 2560 and 6848, weights from HBM) at the row counts
+// that fill one round. The larger tiles do more work per byte they stage, the smaller ones leave
+// fewer CUs idle: 64 x 64 runs 333 x 2560 x 6848 in 24 us (240 tiles) where 128 x 160 took 62 (48
+// tiles), 96 x 128 runs q|k|v|gate of 333 rows in 24 us; from ~1300 rows on the four-wave tiles
+// fill the chip and their larger wave blocks win (1848 x 2560 x 2560: 30 us against 31).
+struct RingTile {
+  int tile;
+  double ktile_us, fixed_us;
+};
+constexpr RingTile kRingTiles[] = {{18, 0.158, 5.5}, {19, 0.166, 6.4}, {20, 0.219, 6.3}, {21, 0.275, 8.8}, {22, 0.225, 9.2},
+                                   {23, 0.290, 9.5}, {24, 0.345, 10.0}, {25, 0.450, 9.5}, {26, 0.545, 9.5}};
+// The four-wave tiles in the same terms: tile area / (rate x this) per K tile, a first round's and a
+// further round's extra (the next tile's loads overlap a persistent round's output), and what the
+// q|k|v store adds to its launch.
+constexpr double kAreaPerUs = 48600.0, kFirstRoundUs = 11.0, kNextRoundUs = 5.0, kQkStoreUs = 9.0;
+
+bool ring_allowed(int tile, int k, int epilogue) {
+  const TileShape t = kTiles[tile];
+  if (!t.ring || k / kBK < t.stages) return false;
+  return epilogue == IRIS_EPI_NONE || (epilogue == IRIS_EPI_SILU_MUL && t.swiglu()) ||
+         (epilogue == kEpiQkRope && t.bn == 128);
+}
+
+long launch_rounds(const TileShape& t, const int* m, int groups, int n, int cus) {
+  long tiles = 0;
+  for (int i = 0; i < groups; ++i) tiles += static_cast<long>((m[i] + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+  return (tiles + cus - 1) / cus;
+}
+
+double four_wave_us(int tile, const int* m, int groups, int n, int k) {
+  double rate = 1.0;
+  for (const Candidate& c : kCandidates)
+    if (c.tile == tile) rate = c.rate;
+  const TileShape t = kTiles[tile];
+  const long rounds = launch_rounds(t, m, groups, n, device_cus());
+  return rounds * (k / kBK) * (t.bm * t.bn / (rate * kAreaPerUs)) + kFirstRoundUs + (rounds - 1) * kNextRoundUs;
+}
+
+// The ring tile that runs the launch in less than `us`, or -1.
+int pick_ring(const int* m, int groups, int n, int k, int epilogue, double us) {
+  int best = -1;
+  for (const RingTile& r : kRingTiles) {
+    if (!ring_allowed(r.tile, k, epilogue)) continue;
+    const double cost =
+        launch_rounds(kTiles[r.tile], m, groups, n, device_cus()) * (k / kBK * r.ktile_us + r.fixed_us);
+    if (cost < us) best = r.tile, us = cost;
+  }
+  return best;
 }
 
 // per thread: a forced tile never changes another thread's launches
@@ -1501,7 +1850,7 @@ int gemm_part(int groups, const void* const* a, const void* const* b, const floa
 }
 
 int launch_args(GemmArgs& args, int c_dtype, int epilogue, int tile, hipStream_t stream) {
-  static_assert(kNumTiles == 18, "one case per tile shape");
+  static_assert(kNumTiles == 27, "one case per tile shape");
   switch (tile) {
 #define IRIS_TILE_CASE(I) \
   case I:                 \
@@ -1524,6 +1873,15 @@ int launch_args(GemmArgs& args, int c_dtype, int epilogue, int tile, hipStream_t
     IRIS_TILE_CASE(15)
     IRIS_TILE_CASE(16)
     IRIS_TILE_CASE(17)
+    IRIS_TILE_CASE(18)
+    IRIS_TILE_CASE(19)
+    IRIS_TILE_CASE(20)
+    IRIS_TILE_CASE(21)
+    IRIS_TILE_CASE(22)
+    IRIS_TILE_CASE(23)
+    IRIS_TILE_CASE(24)
+    IRIS_TILE_CASE(25)
+    IRIS_TILE_CASE(26)
 #undef IRIS_TILE_CASE
     default:
       return fail(IRIS_E_INVALID, "gemm: no tile shape %d", tile);
@@ -1572,6 +1930,14 @@ extern "C" int iris_gemm_bf16_grouped(int groups, const void* const* a, const vo
   for (int i = 0; i < groups; ++i)
     IRIS_REQUIRE(static_cast<long>(m[i]) * lda < (1L << 30), "gemm: activation above 2 GiB (32-bit byte offsets)");
   const SplitPlan plan = plan_split(m, groups, n, epilogue, g_forced_tile);
+  if (g_forced_tile < 0 && mfma16_family(epilogue)) {
+    const double us = plan.n1 == 0 ? four_wave_us(plan.tile1, m, groups, n, k)
+                                   : four_wave_us(plan.tile1, m, groups, plan.n1, k) +
+                                         four_wave_us(plan.tile2, m, groups, n - plan.n1, k) - kFirstRoundUs + kNextRoundUs;
+    const int ring = pick_ring(m, groups, n, k, epilogue, us);
+    if (ring >= 0)
+      return gemm_part(groups, a, b, bias, c, m, c_dtype, n, k, lda, ldb, ldc, epilogue, ring, stream);
+  }
   if (plan.n1 == 0)
     return gemm_part(groups, a, b, bias, c, m, c_dtype, n, k, lda, ldb, ldc, epilogue,
                      pick_tile(m, groups, n, epilogue, g_forced_tile), stream);
@@ -1664,6 +2030,17 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
   qk.eps = eps;
   qk.vt = static_cast<bf16*>(vt);
   qk.n_vt = static_cast<int>(n_vt);
+  // few rows: all columns as one launch of 128-wide ring tiles (a head, or 128 plain columns, each)
+  int ring = -1;
+  if (g_forced_tile < 0) {
+    double us = four_wave_us(kQkRopeTile, m, groups, n < n_qkv ? n : n_qkv, k) + kQkStoreUs;
+    if (n > n_qkv) us += four_wave_us(pick_tile(m, groups, n - n_qkv, IRIS_EPI_NONE, -1), m, groups, n - n_qkv, k);
+    ring = pick_ring(m, groups, n, k, kEpiQkRope, us);
+  } else if (ring_allowed(g_forced_tile, k, kEpiQkRope)) {
+    ring = g_forced_tile;
+  }
+  if (ring >= 0)
+    return gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, ring, stream, &qk);
   if (n <= n_qkv)
     return gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, kQkRopeTile, stream, &qk);
   // the columns after the V heads (the gate columns of a q | k | v | gate weight) are a plain

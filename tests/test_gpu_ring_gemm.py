@@ -1,0 +1,128 @@
+"""The small-tile ring GEMM (`gemm_ring_kernel`, tiles 18 to 26): every epilogue at the edges of its
+tiles, of its ring and of its K loop. Its sums run in the order of the four-wave kernel on the same
+MFMA, so every comparison is exact: against the 256 x 256 or 128 x 160 four-wave tile, which the
+other tests compare with FP32 references."""
+
+import pytest
+import torch
+
+from iris_mi355x import _lib
+from iris_mi355x import kernels as K
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# tile -> (rows, columns, K tiles in the ring)
+RING = {18: (32, 64, 8), 19: (64, 64, 8), 20: (96, 64, 7), 21: (128, 64, 6), 22: (32, 128, 7), 23: (64, 128, 6),
+        24: (96, 128, 5), 25: (128, 128, 4), 26: (192, 128, 3)}
+
+
+def forced(tile, fn):
+    _lib.call("iris_gemm_force_tile", tile)
+    try:
+        return fn()
+    finally:
+        _lib.call("iris_gemm_force_tile", -1)
+
+
+def randn(g, *shape, scale=1.0):
+    return (scale * torch.randn(*shape, generator=g, device=DEV)).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("tile", RING)
+@pytest.mark.parametrize("extra_k", [0, 1, 2, 5])
+@pytest.mark.parametrize("rows,cols", [(0, 1), (1, 0), (-1, -1), (None, None)])
+def test_ring_tile_edges(tile, extra_k, rows, cols):
+    """One row or column unit past or short of whole tiles, a single row, K loops of exactly the ring
+    and of an odd and even number of tiles more; BF16 and FP32 output, bias, padded row strides."""
+    bm, bn, stages = RING[tile]
+    m = 1 if rows is None else 2 * bm + rows
+    n = 4 if cols is None else 2 * bn + 4 * cols
+    k = 64 * (stages + extra_k)
+    g = torch.Generator(device=DEV).manual_seed(40 + extra_k)
+    x, w = randn(g, m, k + 8)[:, :k], randn(g, n, k, scale=0.05)
+    bias = torch.randn(n, generator=g, device=DEV)
+    for kwargs in ({}, {"out_dtype": torch.float32}):
+        for b in (None, bias):
+            got = forced(tile, lambda: K.linear(x, w, b, **kwargs))
+            want = forced(15, lambda: K.linear(x, w, b, **kwargs))
+            assert torch.equal(got, want)
+    prod = x.float().cpu() @ w.float().cpu().T  # k <= 832 products of N(0, 0.05): FP32 sums within 1e-4
+    torch.testing.assert_close(forced(tile, lambda: K.linear(x, w, out_dtype=torch.float32)).cpu(), prod, rtol=1e-4,
+                               atol=1e-4)
+
+
+@pytest.mark.parametrize("tile", [t for t, (_, bn, _) in RING.items() if bn == 128])
+@pytest.mark.parametrize("m,n", [(1, 64), (97, 320), (333, 448)])
+def test_ring_swiglu(tile, m, n):
+    g = torch.Generator(device=DEV).manual_seed(41)
+    x, w = randn(g, m, 576), randn(g, n, 576, scale=0.05)
+    for dtype in (torch.bfloat16, torch.float32):
+        got = forced(tile, lambda: K.linear(x, w, swiglu=True, out_dtype=dtype))
+        assert torch.equal(got, forced(16, lambda: K.linear(x, w, swiglu=True, out_dtype=dtype)))
+
+
+@pytest.mark.parametrize("tile", [18, 20, 25])
+@pytest.mark.parametrize("rows", [(60, 154), (1, 1), (64, 0)])
+def test_ring_two_groups(tile, rows):
+    g = torch.Generator(device=DEV).manual_seed(42)
+    xs, ws = [randn(g, r, 640) for r in rows], [randn(g, 260, 640, scale=0.05) for _ in rows]
+    outs = [[torch.empty(r, 260, device=DEV, dtype=torch.bfloat16) for r in rows] for _ in range(2)]
+    forced(tile, lambda: K.linear_grouped(xs, ws, None, outs[0]))
+    forced(16, lambda: K.linear_grouped(xs, ws, None, outs[1]))
+    for got, want in zip(*outs):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tile", [t for t, (_, bn, _) in RING.items() if bn == 128])
+@pytest.mark.parametrize("heads,kv_heads,tokens,batch,gate", [(3, 1, (37,), 2, True), (2, 2, (60, 77), 1, False),
+                                                             (4, 2, (256,), 2, True), (2, 1, (256, 256), 1, True)])
+def test_ring_qk_store(tile, heads, kv_heads, tokens, batch, gate):
+    """The q | k | v (| gate) store on ring tiles writes what the plain product followed by
+    qkv_prepare writes and nothing else: ragged batch items, two streams, and with whole 256-row
+    items the V heads transposed too."""
+    g = torch.Generator(device=DEV).manual_seed(43)
+    n_qkv = (heads + 2 * kv_heads) * 128
+    n = n_qkv + (128 * heads if gate else 0)
+    v_col, k = (heads + kv_heads) * 128, 512
+    offsets = [tokens[1], 0] if len(tokens) == 2 else [0]
+    n_pad = (sum(tokens) + 63) // 64 * 64 + 64
+    cos, sin = (torch.randn(n_pad, 64, generator=g, device=DEV) for _ in range(2))
+    xs, ws = [randn(g, batch * t, k) for t in tokens], [randn(g, n, k, scale=0.05) for _ in tokens]
+    gains = [[1 + 0.1 * torch.randn(128, generator=g, device=DEV) for _ in tokens] for _ in range(2)]
+
+    def buffers():
+        return [torch.full((batch, h, *s), 3.0, device=DEV, dtype=torch.bfloat16)
+                for h, s in ((heads, (n_pad, 128)), (kv_heads, (n_pad, 128)), (kv_heads, (128, n_pad)))]
+
+    q_ref, k_ref, vt_ref = buffers()
+    plain = [forced(16, lambda x=x, w=w: K.linear(x, w)) for x, w in zip(xs, ws)]
+    for out, qw, kw, t, off in zip(plain, *gains, tokens, offsets):
+        K.qkv_prepare(out.view(batch, t, n), qw, kw, cos, sin, 1e-6, heads, kv_heads, q_ref, k_ref, vt_ref, 0,
+                      heads * 128, v_col, off)
+    for with_vt in (False, True) if all(t % 256 == 0 for t in tokens) else (False,):
+        q, key, vt = buffers()
+        outs = [torch.full((batch * t, n), 5.0, device=DEV, dtype=torch.bfloat16) for t in tokens]
+        forced(tile, lambda: K.linear_qk_rope(xs, ws, outs, *gains, cos, sin, 1e-6, heads, kv_heads, q, key,
+                                              list(tokens), offsets, vt=vt if with_vt else None))
+        assert torch.equal(q, q_ref) and torch.equal(key, k_ref)
+        assert torch.equal(vt, vt_ref) if with_vt else torch.all(vt == 3.0)
+        first = n_qkv if with_vt else v_col
+        for out, ref in zip(outs, plain):
+            assert torch.equal(out[:, first:], ref[:, first:]) and torch.all(out[:, :first] == 5.0)
+
+
+def test_ring_refuses_a_k_loop_shorter_than_its_ring():
+    x, w = torch.zeros(8, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(64, 128, device=DEV, dtype=torch.bfloat16)
+    with pytest.raises(Exception, match="ring"):
+        forced(19, lambda: K.linear(x, w))
+    assert torch.all(K.linear(x, w) == 0)  # the automatic choice takes another tile
+
+
+@pytest.mark.parametrize("n,k,swiglu", [(2560, 2560, False), (13696, 2560, True), (2560, 6848, False)])
+def test_automatic_choice_over_row_counts_is_row_independent(n, k, swiglu):
+    """A row's result does not depend on how many rows the call has, so on which tile runs it."""
+    g = torch.Generator(device=DEV).manual_seed(44)
+    x, w = randn(g, 1500, k), randn(g, n, k, scale=0.02)
+    whole = K.linear(x, w, swiglu=swiglu)
+    for m in (1, 40, 130, 333, 520, 900):
+        assert torch.equal(K.linear(x[:m], w, swiglu=swiglu), whole[:m])
