@@ -311,6 +311,9 @@ class HipIris:
             "qp": e(B, px.num_heads, l_pad, HEAD_DIM), "kp": e(B, px.num_heads, l_pad, HEAD_DIM),
             "vtp": torch.zeros(B, px.num_heads, HEAD_DIM, l_pad, device=dev, dtype=bf16),
         }
+        # [B, 1, D] views of every block's six modulation vectors, made once with the tables
+        ws["mod_views"] = {name: [[block[:, c * D:(c + 1) * D].unsqueeze(1) for c in range(6)] for block in ws[name]]
+                           for name in ("mods_img", "mods_txt")}
         # one batch item: the dual-stream residuals are the single-stream buffer's text and image
         # rows, so joining the streams (and the last block's image rows) moves nothing
         ws["joined_in_place"] = B == 1
@@ -485,8 +488,7 @@ class HipIris:
             self._single_block(ws, blk, B, T, Lp, N, not self.cfg.text_out(index), False, None)
 
     def _mods(self, ws: dict, table: str, index: int, chunk: int) -> torch.Tensor:
-        D = self.cfg.hidden_size
-        return ws[table][index][:, chunk * D:(chunk + 1) * D].unsqueeze(1)
+        return ws["mod_views"][table][index][chunk]
 
     def _dual_block(self, ws: dict, blk: dict, B: int, T: int, Lp: int, N: int, h_ready: bool,
                     nxt: dict | None) -> None:

@@ -32,8 +32,9 @@ class _Check:
 
     def __init__(self, op: str, *tensors: torch.Tensor | None):
         self.op = op
-        if any(t is not None and t.device.type != "cuda" for t in tensors):
-            raise ValueError(f"{op}: the HIP kernels need GPU tensors (there is no CPU path)")
+        for t in tensors:
+            if t is not None and not t.is_cuda:
+                raise ValueError(f"{op}: the HIP kernels need GPU tensors (there is no CPU path)")
 
     def __call__(self, ok: bool, what: str) -> "_Check":
         if not ok:
@@ -41,20 +42,23 @@ class _Check:
         return self
 
     def fp32(self, **tensors: torch.Tensor) -> "_Check":
-        for name, t in tensors.items():
-            self(t.dtype == torch.float32 and t.is_contiguous(), f"{name} must be contiguous FP32 (got {t.dtype})")
+        for name, t in tensors.items():  # (a message is formatted only when it is needed)
+            if t.dtype != torch.float32 or not t.is_contiguous():
+                self(False, f"{name} must be contiguous FP32 (got {t.dtype})")
         return self
 
     def gains(self, width: int, **gains: torch.Tensor) -> "_Check":
         """Per-channel FP32 vectors of ``width`` entries (RMSNorm gains)."""
         self.fp32(**gains)
         for name, g in gains.items():
-            self(g.numel() == width, f"{name}: gain width {g.numel()} does not match the {width} channels")
+            if g.numel() != width:
+                self(False, f"{name}: gain width {g.numel()} does not match the {width} channels")
         return self
 
     def bf16(self, **tensors: torch.Tensor) -> "_Check":
         for name, t in tensors.items():
-            self(t.dtype == torch.bfloat16 and t.is_contiguous(), f"{name} must be contiguous BF16 (got {t.dtype})")
+            if t.dtype != torch.bfloat16 or not t.is_contiguous():
+                self(False, f"{name} must be contiguous BF16 (got {t.dtype})")
         return self
 
 
