@@ -797,9 +797,13 @@ extern "C" int iris_flash_attn(const void* q, const void* k, const void* vt, int
   // ring (one per CU; 230 of them cover a 4352-token sequence) on the 16 x 16 x 32 MFMA when
   // their rounds over the CUs are at least 80% full (variant 5; the 32 x 32 x 16 form, variant 4,
   // was 9-11% faster than variant 1 there, and variant 5 took the step 0.15-0.2 ms below variant
-  // 4); else 32-key tiles staged through registers in three 4-wave workgroups per CU (variant 1:
-  // 168 VGPRs; small grids spread over more CUs). One query head per K/V head (the pixel stage):
-  // 64-key tiles in a 2-stage ring. Each measured fastest at its shapes.
+  // 4). Other lengths take 4-wave workgroups, which spread over more CUs: 64-key tiles in a 2-stage
+  // ring, on the 32 x 32 x 16 MFMA (variant 2) while one item's workgroups fit one round of the CUs,
+  // else on the 16 x 16 x 32 one (variant 6), and for a few tiles 32-key ones staged through
+  // registers (variant 1). One item, us, variant 1 / 2 / 6 / 5: 154 tokens 11.0 / 11.0 / 11.5 /
+  // 21, 333: 14.9 / 14.0 / 15.1 / 28, 1280: 34.8 / 29.5 / 31.6 / 57, 1632: 43 / 38 / 39 / 69, 2560:
+  // 87 / 76 / 74 / 99, 3200: 115 / 105 / 99 / 121, 4096: 217 / 195 / 192 / 162; two items at 2560:
+  // 167 / 150 / 145 / 208. One query head per K/V head (the pixel stage): variant 2.
   // The choice depends on one batch item's shape only: variant 5 rounds differently from
   // variant 1, and a row's result must not depend on the other items of its batch.
   int variant = g_attn_variant;
@@ -809,7 +813,10 @@ extern "C" int iris_flash_attn(const void* q, const void* k, const void* vt, int
       const int cus = device_cus();
       const long wide = static_cast<long>(kv_heads) * (group / 4) * ((n + 95) / 96);
       const long rounds = (wide + cus - 1) / cus;
-      if (wide >= 0.8 * rounds * cus) variant = 5;
+      if (wide >= 0.8 * rounds * cus)
+        variant = 5;
+      else if (n > 192)  // three 64-key tiles
+        variant = static_cast<long>(kv_heads) * (group / 4) * ((n + 31) / 32) <= cus ? 2 : 6;
     }
   }
   const Variant v = kVariants[variant];
