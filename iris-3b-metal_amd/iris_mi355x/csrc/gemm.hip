@@ -1655,6 +1655,7 @@ constexpr int kSquare = 0;  // the 256 x 256 candidate of the 16 x 16 x 32 famil
 // 256 x 256 tile of the family of the plain GEMM, so its outputs are bitwise those of
 // iris_gemm_bf16 followed by iris_qkv_prepare.
 constexpr int kQkRopeTile = 16;
+constexpr int kQkPairTile = 13;  // the gate columns' tile in one launch with that store
 static_assert(kCandidates[kSquare].tile == 16, "256 x 256 16 x 16 x 32 tile");
 
 // Estimated time of one launch with candidate c (arbitrary units: tile area / rate per round).
@@ -1751,31 +1752,72 @@ bool ring_allowed(int tile, int k, int epilogue) {
          (epilogue == kEpiQkRope && t.bn == 128);
 }
 
-long launch_rounds(const TileShape& t, const int* m, int groups, int n, int cus) {
+long launch_tiles(const TileShape& t, const int* m, int groups, int n) {
   long tiles = 0;
   for (int i = 0; i < groups; ++i) tiles += static_cast<long>((m[i] + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
-  return (tiles + cus - 1) / cus;
+  return tiles;
 }
 
-double four_wave_us(int tile, const int* m, int groups, int n, int k) {
+// K loop of one four-wave tile.
+double four_wave_tile_us(int tile, int k) {
   double rate = 1.0;
   for (const Candidate& c : kCandidates)
     if (c.tile == tile) rate = c.rate;
-  const TileShape t = kTiles[tile];
-  const long rounds = launch_rounds(t, m, groups, n, device_cus());
-  return rounds * (k / kBK) * (t.bm * t.bn / (rate * kAreaPerUs)) + kFirstRoundUs + (rounds - 1) * kNextRoundUs;
+  return (k / kBK) * (kTiles[tile].bm * kTiles[tile].bn / (rate * kAreaPerUs));
 }
 
-// The ring tile that runs the launch in less than `us`, or -1.
-int pick_ring(const int* m, int groups, int n, int k, int epilogue, double us) {
+double four_wave_us(int tile, const int* m, int groups, int n, int k) {
+  const int cus = device_cus();
+  const long rounds = (launch_tiles(kTiles[tile], m, groups, n) + cus - 1) / cus;
+  return rounds * four_wave_tile_us(tile, k) + kFirstRoundUs + (rounds - 1) * kNextRoundUs;
+}
+
+// Two GEMMs of n1 and n2 columns in one launch: their tiles follow each other on the CUs, so partial
+// rounds of the first are filled by the second. `extra1` us per tile of the first (its store).
+double pair_us(int tile1, int n1, double extra1, int tile2, int n2, const int* m, int groups, int k) {
+  const double t1 = four_wave_tile_us(tile1, k) + extra1, t2 = four_wave_tile_us(tile2, k), longest = t1 > t2 ? t1 : t2;
+  const double work = (launch_tiles(kTiles[tile1], m, groups, n1) * t1 + launch_tiles(kTiles[tile2], m, groups, n2) * t2) /
+                      device_cus();
+  return (work + 0.5 * t2 > longest ? work + 0.5 * t2 : longest) + kFirstRoundUs;
+}
+
+// The ring tile that runs the launch in less than `us` (which it then lowers to its time), or -1.
+int pick_ring(const int* m, int groups, int n, int k, int epilogue, double& us) {
   int best = -1;
+  const int cus = device_cus();
   for (const RingTile& r : kRingTiles) {
     if (!ring_allowed(r.tile, k, epilogue)) continue;
-    const double cost =
-        launch_rounds(kTiles[r.tile], m, groups, n, device_cus()) * (k / kBK * r.ktile_us + r.fixed_us);
+    const long rounds = (launch_tiles(kTiles[r.tile], m, groups, n) + cus - 1) / cus;
+    const double cost = rounds * (k / kBK * r.ktile_us + r.fixed_us);
     if (cost < us) best = r.tile, us = cost;
   }
   return best;
+}
+
+// The launch plan of one GEMM on the 16 x 16 x 32 MFMA: the four-wave plan, one launch of ring tiles,
+// or whole rounds of 256 x 256 tiles with the columns left over on ring tiles (1280 x 13696 SwiGLU: 255
+// tiles and 640 columns, 79 us against 94 for two half-empty rounds of 192 x 256). The same sums
+// whichever is taken.
+SplitPlan plan_mfma16(const int* m, int groups, int n, int k, int epilogue) {
+  SplitPlan plan = plan_split(m, groups, n, epilogue, -1);
+  double us = plan.n1 == 0 ? four_wave_us(plan.tile1, m, groups, n, k)
+                           : four_wave_us(plan.tile1, m, groups, plan.n1, k) +
+                                 four_wave_us(plan.tile2, m, groups, n - plan.n1, k) - kFirstRoundUs + kNextRoundUs;
+  const int ring = pick_ring(m, groups, n, k, epilogue, us);
+  if (ring >= 0) plan = SplitPlan{0, ring, ring};
+  const int square = kCandidates[kSquare].tile;
+  const long row_tiles = launch_tiles(kTiles[square], m, groups, kTiles[square].bn);
+  for (long rounds = 1; row_tiles > 0; ++rounds) {
+    const long n1 = rounds * device_cus() / row_tiles * 256;
+    if (n1 >= n) break;
+    if (n1 == 0) continue;
+    const double first = four_wave_us(square, m, groups, static_cast<int>(n1), k);
+    if (first >= us) break;
+    double rest = us - first;
+    const int tail = pick_ring(m, groups, n - static_cast<int>(n1), k, epilogue, rest);
+    if (tail >= 0) plan = SplitPlan{static_cast<int>(n1), square, tail}, us = first + rest;
+  }
+  return plan;
 }
 
 // per thread: a forced tile never changes another thread's launches
@@ -1822,7 +1864,7 @@ int make_args(GemmArgs& args, int groups, const void* const* a, const void* cons
 // (256 x 256, then 288 x 160).
 bool has_pair(int tile1, int epi1, int tile2, int epi2) {
   return (tile1 == 16 && epi1 == IRIS_EPI_SILU_MUL && tile2 == 17 && epi2 == IRIS_EPI_SILU_MUL) ||
-         (tile1 == kQkRopeTile && epi1 == kEpiQkRope && tile2 == 13 && epi2 == IRIS_EPI_NONE);
+         (tile1 == kQkRopeTile && epi1 == kEpiQkRope && tile2 == kQkPairTile && epi2 == IRIS_EPI_NONE);
 }
 
 int launch_pair(const GemmArgs& a1, int epi1, const GemmArgs& a2, hipStream_t stream) {
@@ -1929,18 +1971,15 @@ extern "C" int iris_gemm_bf16_grouped(int groups, const void* const* a, const vo
   IRIS_REQUIRE(static_cast<long>(n) * ldb < (1L << 30), "gemm: weight above 2 GiB (32-bit byte offsets)");
   for (int i = 0; i < groups; ++i)
     IRIS_REQUIRE(static_cast<long>(m[i]) * lda < (1L << 30), "gemm: activation above 2 GiB (32-bit byte offsets)");
-  const SplitPlan plan = plan_split(m, groups, n, epilogue, g_forced_tile);
-  if (g_forced_tile < 0 && mfma16_family(epilogue)) {
-    const double us = plan.n1 == 0 ? four_wave_us(plan.tile1, m, groups, n, k)
-                                   : four_wave_us(plan.tile1, m, groups, plan.n1, k) +
-                                         four_wave_us(plan.tile2, m, groups, n - plan.n1, k) - kFirstRoundUs + kNextRoundUs;
-    const int ring = pick_ring(m, groups, n, k, epilogue, us);
-    if (ring >= 0)
-      return gemm_part(groups, a, b, bias, c, m, c_dtype, n, k, lda, ldb, ldc, epilogue, ring, stream);
-  }
+  SplitPlan plan;
+  if (g_forced_tile >= 0)
+    plan.tile1 = g_forced_tile;
+  else if (mfma16_family(epilogue))
+    plan = plan_mfma16(m, groups, n, k, epilogue);
+  else
+    plan.tile1 = pick_tile(m, groups, n, epilogue, -1);
   if (plan.n1 == 0)
-    return gemm_part(groups, a, b, bias, c, m, c_dtype, n, k, lda, ldb, ldc, epilogue,
-                     pick_tile(m, groups, n, epilogue, g_forced_tile), stream);
+    return gemm_part(groups, a, b, bias, c, m, c_dtype, n, k, lda, ldb, ldc, epilogue, plan.tile1, stream);
   // columns [0, n1) and [n1, n): weight rows, bias entries and output columns of the second part
   // start at n1 (n1 / 2 output columns for SwiGLU); one launch for both where a pair kernel exists
   GemmArgs a1, a2;
@@ -2030,14 +2069,25 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
   qk.eps = eps;
   qk.vt = static_cast<bf16*>(vt);
   qk.n_vt = static_cast<int>(n_vt);
-  // few rows: all columns as one launch of 128-wide ring tiles (a head, or 128 plain columns, each)
-  int ring = -1;
+  // The q | k | v store with the columns after it (the gate) as a second GEMM, in one launch on the
+  // 288 x 160 tile of the pair kernel or in two; or, for few rows, all columns as one launch of
+  // 128-wide ring tiles (a head, or 128 plain columns, each). Measured, K = 2560 and 6400 columns:
+  // 4096 + 300 rows 192 us in two launches (270 and 240 tiles, each a little over or under a round)
+  // against 171 us paired, 2304 rows 111 against 93 us; 1280 rows 94 us in two launches against 56 us
+  // on ring tiles.
+  int ring = -1, tile2 = -1;
   if (g_forced_tile < 0) {
     double us = four_wave_us(kQkRopeTile, m, groups, n < n_qkv ? n : n_qkv, k) + kQkStoreUs;
-    if (n > n_qkv) us += four_wave_us(pick_tile(m, groups, n - n_qkv, IRIS_EPI_NONE, -1), m, groups, n - n_qkv, k);
+    if (n > n_qkv) {
+      tile2 = pick_tile(m, groups, n - n_qkv, IRIS_EPI_NONE, -1);
+      us += four_wave_us(tile2, m, groups, n - n_qkv, k);
+      const double paired = pair_us(kQkRopeTile, n_qkv, kQkStoreUs, kQkPairTile, n - n_qkv, m, groups, k);
+      if (paired < us) tile2 = kQkPairTile, us = paired;
+    }
     ring = pick_ring(m, groups, n, k, kEpiQkRope, us);
-  } else if (ring_allowed(g_forced_tile, k, kEpiQkRope)) {
-    ring = g_forced_tile;
+  } else {
+    tile2 = g_forced_tile;
+    if (ring_allowed(g_forced_tile, k, kEpiQkRope)) ring = g_forced_tile;
   }
   if (ring >= 0)
     return gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, ring, stream, &qk);
@@ -2054,7 +2104,6 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
     b2[i] = b[i] ? static_cast<const bf16*>(b[i]) + static_cast<long>(n_qkv) * ldb : nullptr;
     c2[i] = c[i] ? static_cast<bf16*>(c[i]) + n_qkv : nullptr;
   }
-  const int tile2 = pick_tile(m, groups, n - n_qkv, IRIS_EPI_NONE, g_forced_tile);
   rc = make_args(a2, groups, a, b2, nullptr, c2, m, n - n_qkv, k, lda, ldb, ldc, IRIS_EPI_NONE, tile2, nullptr);
   if (rc != IRIS_OK) return rc;
   return launch_two(a1, kQkRopeTile, kEpiQkRope, a2, tile2, IRIS_EPI_NONE, IRIS_BF16, stream);
