@@ -223,6 +223,17 @@ int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const void* const* 
 int iris_gemv_bf16(const void* w, const float* x, int batch, int n, int k, const float* bias,
                    const float* extra_bias, int n_extra, float* out, int in_act, int out_act, hipStream_t stream);
 
+/* Two such products of the same inputs in one launch (the image and text adaLN cores), arrays of two;
+ * bias and extra_bias entries may be null. */
+int iris_gemv_bf16_pair(const void* const* w, const float* x, int batch, const int* n, int k,
+                        const float* const* bias, const float* const* extra_bias, const int* n_extra,
+                        float* const* out, int in_act, int out_act, hipStream_t stream);
+
+/* iris_timestep_features followed by iris_gemv_bf16 over them (the timestep MLP's first layer) in one
+ * launch: W BF16 [n, 2 half]. */
+int iris_timestep_gemv_bf16(const float* t, const float* freqs, int half, const void* w, int batch, int n,
+                            const float* bias, float* out, int out_act, hipStream_t stream);
+
 /* Sinusoidal timestep features [cos | sin] (src/iris3b/nn/embeddings.py:41-45):
  * out[b, j] = cos(t[b] * freqs[j]), out[b, half + j] = sin(t[b] * freqs[j]). */
 int iris_timestep_features(const float* t, const float* freqs, int batch, int half, float* out,

@@ -7,6 +7,9 @@
 // inputs are activated once per workgroup and reach the registers through LDS. R = 8 where that
 // still gives every CU a workgroup or two (the per-block copies of an output then leave as 32-byte
 // pieces), else 2; figures at launch_rows.
+// One launch runs the image and the text core (they share their inputs), and the first timestep
+// layer computes the sinusoidal features it reads, so the chain is three launches: 51 -> 44 us per
+// denoise step.
 // gemv_kernel: any k and batch whose inputs do not fit the registers (more than 20 chunks per lane).
 // Both add a row's products in the same order, so they agree bit for bit.
 #include "iris_common.hpp"
@@ -18,16 +21,39 @@ constexpr int kMaxBatch = 4;
 constexpr int kRowsPerWave = 2;
 constexpr int kRowsPerBlock = 4 * kRowsPerWave;
 
+// One product over the inputs of a launch.
+struct GemvJob {
+  const bf16* w;
+  int n;
+  const float *bias, *extra;
+  int n_extra;
+  float* out;
+  long out_bstride, out_jstride;
+};
+// A launch: one job, or two on the same inputs (workgroups from `blocks0` on run the second). With
+// freqs the inputs are the timestep features [cos | sin](x[b] freqs) of k / 2 frequencies.
+struct GemvLaunch {
+  GemvJob job[2];
+  int blocks0;
+  const float *x, *freqs;
+  int k, in_act, out_act;
+};
+
 template <int NCH, int NB, int R>
-__global__ __launch_bounds__(256, 2) void gemv_rows_kernel(const bf16* __restrict__ w, const float* __restrict__ x, int n,
-                                                        int k, const float* __restrict__ bias,
-                                                        const float* __restrict__ extra, int n_extra,
-                                                        float* __restrict__ out, long out_bstride, long out_jstride,
-                                                        int in_act, int out_act) {
+__global__ __launch_bounds__(256, 2) void gemv_rows_kernel(GemvLaunch a) {
   constexpr int DEPTH = R < 4 ? R : (NB * NCH > 10 ? 2 : 4);  // rows in flight
   extern __shared__ float xs[];  // NB * k
+  const bool second = static_cast<int>(blockIdx.x) >= a.blocks0;
+  const GemvJob& job = second ? a.job[1] : a.job[0];
+  const bf16* __restrict__ w = job.w;
+  const float* __restrict__ x = a.x;
+  const float* __restrict__ bias = job.bias;
+  const float* __restrict__ extra = job.extra;
+  float* __restrict__ out = job.out;
+  const int n = job.n, k = a.k, n_extra = job.n_extra;
+  const long out_bstride = job.out_bstride, out_jstride = job.out_jstride;
   const int lane = threadIdx.x & 63;
-  const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
+  const int row0 = ((static_cast<int>(blockIdx.x) - (second ? a.blocks0 : 0)) * 4 + (threadIdx.x >> 6)) * R;
   const int chunks = k >> 3;
   bf16x8 wv[DEPTH][NCH];
   auto load_row = [&](int r) {
@@ -40,10 +66,20 @@ __global__ __launch_bounds__(256, 2) void gemv_rows_kernel(const bf16* __restric
   };
 #pragma unroll
   for (int r = 0; r < DEPTH; ++r) load_row(r);
-  for (int i = 4 * threadIdx.x; i < NB * k; i += 4 * 256) {
-    f32x4 v = load4(x + i);
-    if (in_act == IRIS_ACT_SILU) v = f32x4{silu(v[0]), silu(v[1]), silu(v[2]), silu(v[3])};
-    store4(xs + i, v);
+  if (a.freqs) {
+    const int half = k >> 1;
+    for (int i = threadIdx.x; i < NB * half; i += 256) {
+      const int b = i / half, j = i - b * half;
+      const float phase = x[b] * a.freqs[j];
+      xs[b * k + j] = cosf(phase);
+      xs[b * k + half + j] = sinf(phase);
+    }
+  } else {
+    for (int i = 4 * threadIdx.x; i < NB * k; i += 4 * 256) {
+      f32x4 v = load4(x + i);
+      if (a.in_act == IRIS_ACT_SILU) v = f32x4{silu(v[0]), silu(v[1]), silu(v[2]), silu(v[3])};
+      store4(xs + i, v);
+    }
   }
   __syncthreads();
   if (row0 >= n) return;
@@ -91,7 +127,7 @@ __global__ __launch_bounds__(256, 2) void gemv_rows_kernel(const bf16* __restric
 #pragma unroll
     for (int r = 1; r < R; ++r) v = rr == r ? y[b][r] : v;
     if (bias) v += bv;
-    if (out_act == IRIS_ACT_SILU) v = silu(v);
+    if (a.out_act == IRIS_ACT_SILU) v = silu(v);
     if (n_extra == 0) {
       if (lane < R) out[b * out_bstride + row] = v;
     } else {
@@ -149,17 +185,6 @@ __global__ __launch_bounds__(256) void gemv_kernel(const bf16* __restrict__ w, c
   }
 }
 
-struct GemvArgs {
-  const bf16* w;
-  const float* x;
-  int n, k;
-  const float *bias, *extra;
-  int n_extra;
-  float* out;
-  long out_bstride, out_jstride;
-  int in_act, out_act;
-};
-
 // Measured on one box, us per call (TB/s of weight), HIP-graph replays with every weight from HBM:
 //                                    batch 1        2             3             4
 //   15360 x 2560, 24 bias rows, before 28.8 (2.7)   48.2 (1.6)    73.2 (1.1)    99.4 (0.8)
@@ -169,38 +194,75 @@ struct GemvArgs {
 // (before: gemv_kernel, whose input reads from LDS grew with the batch). A copy of this size class
 // moves 4.8 TB/s; batch 4 has two waves per SIMD to hide its latency (250 VGPRs).
 template <int NCH, int NB>
-void launch_rows(const GemvArgs& a, hipStream_t stream) {
+void launch_rows(GemvLaunch& a, int jobs, hipStream_t stream) {
   const size_t lds = static_cast<size_t>(NB) * a.k * sizeof(float);
-  const bool many = a.n >= 4 * 8 * device_cus();  // 8 rows per wave still fill the CUs
+  const int rows = a.job[0].n + (jobs > 1 ? a.job[1].n : 0);
+  const bool many = rows >= 4 * 8 * device_cus();  // 8 rows per wave still fill the CUs
   const int per_wg = 4 * (many ? 8 : 2);
-  const dim3 grid((a.n + per_wg - 1) / per_wg);
+  a.blocks0 = (a.job[0].n + per_wg - 1) / per_wg;
+  const dim3 grid(a.blocks0 + (jobs > 1 ? (a.job[1].n + per_wg - 1) / per_wg : 0));
   if (many)
-    gemv_rows_kernel<NCH, NB, 8><<<grid, 256, lds, stream>>>(a.w, a.x, a.n, a.k, a.bias, a.extra, a.n_extra, a.out,
-                                                             a.out_bstride, a.out_jstride, a.in_act, a.out_act);
+    gemv_rows_kernel<NCH, NB, 8><<<grid, 256, lds, stream>>>(a);
   else
-    gemv_rows_kernel<NCH, NB, 2><<<grid, 256, lds, stream>>>(a.w, a.x, a.n, a.k, a.bias, a.extra, a.n_extra, a.out,
-                                                             a.out_bstride, a.out_jstride, a.in_act, a.out_act);
+    gemv_rows_kernel<NCH, NB, 2><<<grid, 256, lds, stream>>>(a);
 }
 
 template <int NCH>
-bool launch_batch(const GemvArgs& a, int nb, hipStream_t stream) {
+bool launch_batch(GemvLaunch& a, int jobs, int nb, hipStream_t stream) {
   switch (nb) {
-    case 1: launch_rows<NCH, 1>(a, stream); return true;
-    case 2: launch_rows<NCH, 2>(a, stream); return true;
-    case 3: if constexpr (3 * NCH <= 20) { launch_rows<NCH, 3>(a, stream); return true; } break;
-    case 4: if constexpr (4 * NCH <= 20) { launch_rows<NCH, 4>(a, stream); return true; } break;
+    case 1: launch_rows<NCH, 1>(a, jobs, stream); return true;
+    case 2: launch_rows<NCH, 2>(a, jobs, stream); return true;
+    case 3: if constexpr (3 * NCH <= 20) { launch_rows<NCH, 3>(a, jobs, stream); return true; } break;
+    case 4: if constexpr (4 * NCH <= 20) { launch_rows<NCH, 4>(a, jobs, stream); return true; } break;
   }
   return false;
 }
 
 // The register form where it is instantiated (the chunks per lane of the widths in use: 256, 2560).
-bool launch_registers(const GemvArgs& a, int nb, hipStream_t stream) {
-  if (!aligned(a.x, 16)) return false;
+bool launch_registers(GemvLaunch& a, int jobs, int nb, hipStream_t stream) {
+  if (!a.freqs && !aligned(a.x, 16)) return false;
   const int nch = (a.k / 8 + kWave - 1) / kWave;
-  if (nch == 1) return launch_batch<1>(a, nb, stream);
-  if (nch == 5) return launch_batch<5>(a, nb, stream);
+  if (nch == 1) return launch_batch<1>(a, jobs, nb, stream);
+  if (nch == 5) return launch_batch<5>(a, jobs, nb, stream);
   return false;
 }
+
+// `jobs` products of all batch items, four items per launch; the jobs' outputs are [n_extra,] batch, n.
+int gemv_launch(const GemvLaunch& whole, int jobs, int batch, hipStream_t stream) {
+  for (int b0 = 0; b0 < batch; b0 += kMaxBatch) {
+    const int nb = batch - b0 < kMaxBatch ? batch - b0 : kMaxBatch;
+    GemvLaunch a = whole;
+    a.x += static_cast<long>(b0) * (a.freqs ? 1 : a.k);
+    for (int j = 0; j < jobs; ++j) {
+      a.job[j].out_bstride = a.job[j].n;
+      a.job[j].out_jstride = static_cast<long>(batch) * a.job[j].n;
+      a.job[j].out += static_cast<long>(b0) * a.job[j].n;
+    }
+    if (!launch_registers(a, jobs, nb, stream)) {
+      if (a.freqs) return fail(IRIS_E_UNSUPPORTED, "timestep_gemv: at most 256 frequencies");
+      for (int j = 0; j < jobs; ++j) {
+        const GemvJob& g = a.job[j];
+        const dim3 grid((g.n + kRowsPerBlock - 1) / kRowsPerBlock);
+        const size_t lds = static_cast<size_t>(nb) * a.k * sizeof(float);
+        gemv_kernel<<<grid, 256, lds, stream>>>(g.w, a.x, nb, g.n, a.k, g.bias, g.extra, g.n_extra, g.out,
+                                                g.out_bstride, g.out_jstride, a.in_act, a.out_act);
+      }
+    }
+    const int rc = check_launch("gemv");
+    if (rc) return rc;
+  }
+  return IRIS_OK;
+}
+
+int check_job(const GemvJob& job, int k) {
+  IRIS_REQUIRE(job.n > 0 && k > 0 && k % 8 == 0 && k <= 4096, "gemv: need k %% 8 == 0 and k <= 4096");
+  IRIS_REQUIRE(job.n_extra >= 0 && (job.n_extra == 0 || job.extra), "gemv: extra biases missing");
+  IRIS_REQUIRE(job.w && job.out, "gemv: null pointer");
+  IRIS_REQUIRE(aligned(job.w, 16), "gemv: weight must be 16-byte aligned");
+  return IRIS_OK;
+}
+
+bool valid_act(int act) { return act == IRIS_ACT_NONE || act == IRIS_ACT_SILU; }
 
 }  // namespace
 }  // namespace iris
@@ -210,27 +272,49 @@ using namespace iris;
 extern "C" int iris_gemv_bf16(const void* w, const float* x, int batch, int n, int k, const float* bias,
                               const float* extra_bias, int n_extra, float* out, int in_act, int out_act,
                               hipStream_t stream) {
-  IRIS_REQUIRE(batch >= 0 && n > 0 && k > 0 && k % 8 == 0 && k <= 4096, "gemv: need k %% 8 == 0 and k <= 4096");
-  IRIS_REQUIRE(n_extra >= 0 && (n_extra == 0 || extra_bias), "gemv: extra biases missing");
-  IRIS_REQUIRE((in_act == IRIS_ACT_NONE || in_act == IRIS_ACT_SILU) &&
-                   (out_act == IRIS_ACT_NONE || out_act == IRIS_ACT_SILU),
-               "gemv: unknown activation");
-  IRIS_REQUIRE(w && x && out, "gemv: null pointer");
-  IRIS_REQUIRE(aligned(w, 16), "gemv: weight must be 16-byte aligned");
-  const long out_bstride = n;
-  const long out_jstride = static_cast<long>(batch) * n;
-  for (int b0 = 0; b0 < batch; b0 += kMaxBatch) {
-    const int nb = batch - b0 < kMaxBatch ? batch - b0 : kMaxBatch;
-    const GemvArgs args{static_cast<const bf16*>(w), x + static_cast<long>(b0) * k, n, k, bias, extra_bias, n_extra,
-                        out + static_cast<long>(b0) * n, out_bstride, out_jstride, in_act, out_act};
-    if (!launch_registers(args, nb, stream)) {
-      const dim3 grid((n + kRowsPerBlock - 1) / kRowsPerBlock);
-      const size_t lds = static_cast<size_t>(nb) * k * sizeof(float);
-      gemv_kernel<<<grid, 256, lds, stream>>>(args.w, args.x, nb, n, k, bias, extra_bias, n_extra, args.out, out_bstride,
-                                              out_jstride, in_act, out_act);
-    }
-    const int rc = check_launch("gemv");
+  GemvLaunch a{};
+  a.job[0] = GemvJob{static_cast<const bf16*>(w), n, bias, extra_bias, n_extra, out, 0, 0};
+  a.x = x;
+  a.k = k;
+  a.in_act = in_act;
+  a.out_act = out_act;
+  IRIS_REQUIRE(batch >= 0 && x, "gemv: bad batch or input");
+  IRIS_REQUIRE(valid_act(in_act) && valid_act(out_act), "gemv: unknown activation");
+  const int rc = check_job(a.job[0], k);
+  return rc ? rc : gemv_launch(a, 1, batch, stream);
+}
+
+extern "C" int iris_gemv_bf16_pair(const void* const* w, const float* x, int batch, const int* n, int k,
+                                   const float* const* bias, const float* const* extra_bias, const int* n_extra,
+                                   float* const* out, int in_act, int out_act, hipStream_t stream) {
+  IRIS_REQUIRE(w && n && bias && extra_bias && n_extra && out, "gemv: null pointer");
+  IRIS_REQUIRE(batch >= 0 && x, "gemv: bad batch or input");
+  IRIS_REQUIRE(valid_act(in_act) && valid_act(out_act), "gemv: unknown activation");
+  GemvLaunch a{};
+  a.x = x;
+  a.k = k;
+  a.in_act = in_act;
+  a.out_act = out_act;
+  for (int j = 0; j < 2; ++j) {
+    a.job[j] = GemvJob{static_cast<const bf16*>(w[j]), n[j], bias[j], extra_bias[j], n_extra[j], out[j], 0, 0};
+    const int rc = check_job(a.job[j], k);
     if (rc) return rc;
   }
-  return IRIS_OK;
+  return gemv_launch(a, 2, batch, stream);
+}
+
+extern "C" int iris_timestep_gemv_bf16(const float* t, const float* freqs, int half, const void* w, int batch, int n,
+                                       const float* bias, float* out, int out_act, hipStream_t stream) {
+  IRIS_REQUIRE(batch >= 0 && t && freqs && half > 0 && half % 4 == 0 && half <= 256,
+               "timestep_gemv: need 4 to 256 frequencies, a multiple of 4");
+  IRIS_REQUIRE(valid_act(out_act), "gemv: unknown activation");
+  GemvLaunch a{};
+  a.job[0] = GemvJob{static_cast<const bf16*>(w), n, bias, nullptr, 0, out, 0, 0};
+  a.x = t;
+  a.freqs = freqs;
+  a.k = 2 * half;
+  a.in_act = IRIS_ACT_NONE;
+  a.out_act = out_act;
+  const int rc = check_job(a.job[0], a.k);
+  return rc ? rc : gemv_launch(a, 1, batch, stream);
 }

@@ -296,7 +296,7 @@ class HipIris:
             "L": Lp, "N": N, "n_pad": n_pad, "l_pad": l_pad, "grid": (hp, wp),
             "patches": torch.zeros(B * Lp, self.patch_k, device=dev, dtype=bf16),
             "X": e(B * Lp, D, dtype=f32), "Y": e(B * T, D, dtype=f32), "tok": e(B * N, D, dtype=f32),
-            "tfeat": e(B, 256, dtype=f32), "th": e(B, D, dtype=f32), "temb": e(B, D, dtype=f32),
+            "th": e(B, D, dtype=f32), "temb": e(B, D, dtype=f32),
             "mods_img": e(n_img, B, 6 * D, dtype=f32), "mods_txt": e(n_txt, B, 6 * D, dtype=f32),
             "h_tok": e(B * N, D), "qkvg": e(B * N, qkvg_w), "attn": e(B * N, D), "branch": e(B * N, D),
             "hh": e(B * N, self.hidden_pad),
@@ -429,11 +429,10 @@ class HipIris:
 
     def _conditioning(self, ws: dict, t: torch.Tensor) -> None:
         """Timestep embedding, then both shared adaLN cores with every block's bias folded in."""
-        K.timestep_features(t, self.t_freqs, ws["tfeat"])
-        K.gemv(self.t0_w, ws["tfeat"], self.t0_b, ws["th"], out_silu=True)
+        K.timestep_gemv(t, self.t_freqs, self.t0_w, self.t0_b, ws["th"], out_silu=True)
         K.gemv(self.t2_w, ws["th"], self.t2_b, ws["temb"])
-        K.gemv(self.core_img_w, ws["temb"], self.core_img_b, ws["mods_img"], extra_bias=self.img_bias, in_silu=True)
-        K.gemv(self.core_txt_w, ws["temb"], self.core_txt_b, ws["mods_txt"], extra_bias=self.txt_bias, in_silu=True)
+        K.gemv_pair([self.core_img_w, self.core_txt_w], ws["temb"], [self.core_img_b, self.core_txt_b],
+                    [ws["mods_img"], ws["mods_txt"]], [self.img_bias, self.txt_bias], in_silu=True)
 
     @torch.no_grad()
     def block_forward(self, index: int, x: torch.Tensor, text: torch.Tensor, t: torch.Tensor,

@@ -684,6 +684,39 @@ def gemv(
     return out
 
 
+def gemv_pair(weights, x: torch.Tensor, biases, outs, extra_biases, in_silu: bool = False) -> None:
+    """``gemv`` with extra biases of two weights on the same inputs (the image and text adaLN cores)
+    in one launch; same results as the two calls."""
+    batch, k = x.shape
+    for w, b, o, e in zip(weights, biases, outs, extra_biases):
+        check = _Check("gemv_pair", w, x, b, o, e)
+        check(w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] == k, "BF16 contiguous [N, K] weights")
+        check.fp32(x=x, bias=b, extra_bias=e, out=o)
+        check(o.shape == (e.shape[0], batch, w.shape[0]) and e.shape[1] == w.shape[0] and b.numel() == w.shape[0],
+              "bad out or biases")
+    P = L.pointer_array
+    L.call(
+        "iris_gemv_bf16_pair", P([L.ptr(w) for w in weights]), L.ptr(x), batch, L.int_array([w.shape[0] for w in weights]),
+        k, P([L.ptr(b) for b in biases]), P([L.ptr(e) for e in extra_biases]),
+        L.int_array([e.shape[0] for e in extra_biases]), P([L.ptr(o) for o in outs]),
+        L.ACT_SILU if in_silu else L.ACT_NONE, L.ACT_NONE, L.stream(),
+    )
+
+
+def timestep_gemv(t: torch.Tensor, freqs: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, out: torch.Tensor,
+                  out_silu: bool = False) -> torch.Tensor:
+    """``gemv`` over ``timestep_features(t, freqs)`` in one launch (the timestep MLP's first layer)."""
+    n, k = weight.shape
+    check = _Check("timestep_gemv", t, freqs, weight, bias, out)
+    check.fp32(t=t, freqs=freqs, bias=bias, out=out)
+    check(weight.dtype == torch.bfloat16 and weight.is_contiguous() and k == 2 * freqs.numel() and bias.numel() == n,
+          "BF16 contiguous [N, 2 * frequencies] weight")
+    check(out.shape == (t.numel(), n), "bad out")
+    L.call("iris_timestep_gemv_bf16", L.ptr(t), L.ptr(freqs), freqs.numel(), L.ptr(weight), t.numel(), n, L.ptr(bias),
+           L.ptr(out), L.ACT_SILU if out_silu else L.ACT_NONE, L.stream())
+    return out
+
+
 def patchify_embed(x, patch, pix_w, pix_b, pos_x, pos_y, norm_weight, eps, patches, pixels, normed) -> None:
     """Patch matrix for the patch embedder, the embedded pixel stream and its first norm
     (src/iris_metal/model.py:188-189, 208-210)."""

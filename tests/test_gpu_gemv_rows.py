@@ -37,3 +37,33 @@ def test_gemv_rows(n, k, batch, extra):
         # k <= 2560 products of N(0, 0.05) in FP32 (and silu's ~1 ulp reciprocal): 2^-24 sqrt(k) of their sum
         ok = torch.isfinite(want)
         torch.testing.assert_close(out.double()[ok], want[ok], rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("ns,k", [((8200, 37), 256), ((7, 1), 512), ((9000, 8192), 2560), ((40, 24), 520)])
+@pytest.mark.parametrize("batch", [1, 2, 4, 7])
+def test_gemv_pair_is_two_gemvs(ns, k, batch):
+    """Two products in one launch, exactly as two calls (520: the general kernel)."""
+    g = torch.Generator(device=DEV).manual_seed(51)
+    ws = [(0.05 * torch.randn(n, k, generator=g, device=DEV)).to(torch.bfloat16) for n in ns]
+    x = torch.randn(batch, k, generator=g, device=DEV)
+    biases = [torch.randn(n, generator=g, device=DEV) for n in ns]
+    extras = [torch.randn(j, n, generator=g, device=DEV) for j, n in zip((24, 8), ns)]
+    outs = [[torch.full((e.shape[0], batch, n), 7.0, device=DEV) for e, n in zip(extras, ns)] for _ in range(2)]
+    K.gemv_pair(ws, x, biases, outs[0], extras, in_silu=True)
+    for w, b, o, e in zip(ws, biases, outs[1], extras):
+        K.gemv(w, x, b, o, extra_bias=e, in_silu=True)
+    for got, want in zip(*outs):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,half", [(2560, 128), (1, 4), (259, 256), (8195, 100)])
+@pytest.mark.parametrize("batch", [1, 3, 6])
+def test_timestep_gemv_is_features_then_gemv(n, half, batch):
+    g = torch.Generator(device=DEV).manual_seed(52)
+    w = (0.05 * torch.randn(n, 2 * half, generator=g, device=DEV)).to(torch.bfloat16)
+    bias = torch.randn(n, generator=g, device=DEV)
+    t, freqs = 1000 * torch.rand(batch, generator=g, device=DEV), torch.rand(half, generator=g, device=DEV)
+    features, out, want = (torch.empty(batch, m, device=DEV) for m in (2 * half, n, n))
+    K.timestep_gemv(t, freqs, w, bias, out, out_silu=True)
+    K.gemv(w, K.timestep_features(t, freqs, features), bias, want, out_silu=True)
+    assert torch.equal(out, want)
