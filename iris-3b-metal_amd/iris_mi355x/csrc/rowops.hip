@@ -2,10 +2,10 @@
 // residual (optionally fused with the next RMSNorm + modulate), per-head qk-RMSNorm + 2-D
 // RoPE, the V-head transpose, and small row utilities.
 //
-// Layout: one 64-lane wave per D-wide row; lane l owns the 8-element chunks l, l + 64, ...
-// (16-byte BF16 / 32-byte FP32 accesses, 1 KB or 2 KB contiguous per wave instruction), and
-// the row stays in registers between the statistics pass and the output pass, so HBM sees
-// each byte once.
+// Layout: 8-element chunks of a D-wide row (16-byte BF16 / 32-byte FP32 accesses, 1 KB or 2 KB
+// contiguous per wave instruction), chunks l, l + 64, ... in lane l of one wave or (the split forms)
+// one per thread of a workgroup; the row stays in registers between the statistics pass and the
+// output pass, so HBM sees each byte once.
 #include "iris_common.hpp"
 
 namespace iris {
@@ -22,6 +22,8 @@ struct Chunk8<bf16> {
   bf16x8 v;
   __device__ __forceinline__ void load(const bf16* p) { v = *reinterpret_cast<const bf16x8*>(p); }
   __device__ __forceinline__ float operator[](int e) const { return to_f32(v[e]); }
+  // later reads convert the values again (kept in FP32 from the statistics pass on, they spill)
+  __device__ __forceinline__ void reread() { asm volatile("" : "+v"(v)); }
 };
 template <>
 struct Chunk8<float> {
@@ -31,7 +33,44 @@ struct Chunk8<float> {
     b = *reinterpret_cast<const f32x4*>(p + 4);
   }
   __device__ __forceinline__ float operator[](int e) const { return e < 4 ? a[e] : b[e - 4]; }
+  __device__ __forceinline__ void reread() {}
 };
+
+// Arithmetic that the wave-per-row and the workgroup-per-row (split) forms share, spelled out so that
+// they agree bit for bit. A row's squares are summed per 8-element chunk in element order, a lane's
+// chunks in order, and the lanes as wave_sum does; the split form (a wave per 512 columns) passes the
+// chunk sums through LDS and then adds in the same order.
+template <typename C>
+__device__ __forceinline__ float chunk_sq(const C& v) {
+  float ss = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(v[e], v[e], ss);
+  return ss;
+}
+__device__ __forceinline__ float rms_scale(float sum_sq, int width, float eps) {
+  return rsqrtf(sum_sq / static_cast<float>(width) + eps);
+}
+template <int NC>
+__device__ __forceinline__ float split_row_sum(float chunk, float (&part)[NC][kWave], int i, int lane) {
+  if constexpr (NC == 1) return wave_sum(chunk);
+  part[i][lane] = chunk;
+  __syncthreads();
+  float ss = part[0][lane];
+#pragma unroll
+  for (int k = 1; k < NC; ++k) ss += part[k][lane];
+  return wave_sum(ss);
+}
+
+// The split forms run launches of at most this many rows: a wave per row leaves most of the chip idle
+// there and walks its loads, reductions and coefficient reads one after the other, where a workgroup
+// per row has them all in flight at once. With many rows the reductions, which each of a row's waves
+// repeats, cost more than that saves: in the 1024 x 1024 denoise step, at the clocks the GEMMs leave,
+// the gated residual of 4352 rows takes 30.7 us with a wave per row and 34.7 split. us per call at
+// width 2560 with every buffer from HBM, split / wave per row: gated residual with the next norm 333
+// rows 6.8 / 7.7, 1280: 13.4 / 15.8, 1848: 18.9 / 18.8; modulate FP32 333: 4.3 / 5.0, 1280: 7.3 / 7.8,
+// 1848: 10.0 / 9.4; modulate BF16 333: 4.0 / 4.6, 640: 4.9 / 4.6, 4352: 16.2 / 12.3.
+constexpr long kGatedSplitRows = 1792;
+long modulate_split_rows(int x_dtype) { return x_dtype == IRIS_F32 ? 1536 : 512; }
 
 // NC = 8-element chunks each lane holds (width <= NC * 512). A wave issues its row's loads
 // first, reduces, and reads the per-column FP32 coefficients chunk by chunk in the output pass,
@@ -73,13 +112,9 @@ __global__ __launch_bounds__(256) void rms_norm_modulate_kernel(const TI* __rest
   }
   float ss = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int j = lane + i * kWave;
-    if (j < nc)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
-  }
-  const float r = rsqrtf(wave_sum(ss) / static_cast<float>(width) + eps);
+  for (int i = 0; i < NC; ++i)
+    if (lane + i * kWave < nc) ss += chunk_sq(v[i]);
+  const float r = rms_scale(wave_sum(ss), width, eps);
   const long b = row / rows_per_batch;
   TO* o = out + row * width;
 #pragma unroll
@@ -99,19 +134,46 @@ __global__ __launch_bounds__(256) void rms_norm_modulate_kernel(const TI* __rest
         for (int e = 0; e < 8; ++e) m[e] = w[e] * (1.0f + s1[e]);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = (v[i][e] * r) * m[e] + c0[e];
+      for (int e = 0; e < 8; ++e) y[e] = __builtin_fmaf(v[i][e] * r, m[e], c0[e]);
       store8(o + 8 * j, y);
     }
   }
 }
 
+// rms_norm_modulate_kernel with a workgroup of NC waves per row, one chunk per thread.
+template <int NC, typename TI, typename TO>
+__global__ __launch_bounds__(64 * NC) void rms_norm_modulate_split_kernel(const TI* __restrict__ x, TO* __restrict__ out,
+                                                                          const float* __restrict__ weight,
+                                                                          const float* __restrict__ shift,
+                                                                          const float* __restrict__ scale,
+                                                                          long rows_per_batch, int width,
+                                                                          long mod_stride, float eps) {
+  __shared__ float part[NC][kWave];
+  const long row = blockIdx.x;
+  const int lane = threadIdx.x & 63, i = threadIdx.x >> 6, j = threadIdx.x;
+  const bool in = j < width >> 3;
+  const long b = row / rows_per_batch;
+  Chunk8<TI> v;
+  float w[8], s1[8], c0[8];
+  if (in) {
+    v.load(x + row * width + 8 * j);
+    load8(weight + 8 * j, w);
+    load8(scale + b * mod_stride + 8 * j, s1);
+    load8(shift + b * mod_stride + 8 * j, c0);
+  }
+  const float r = rms_scale(split_row_sum<NC>(in ? chunk_sq(v) : 0.0f, part, i, lane), width, eps);
+  if (!in) return;
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = __builtin_fmaf(v[e] * r, w[e] * (1.0f + s1[e]), c0[e]);
+  store8(out + row * width + 8 * j, y);
+}
+
 // residual[r] += gate * rmsnorm(branch[r]) * weight; with next_out, also
 // next_out[r] = rmsnorm(residual[r]) * next_weight * (1 + next_scale) + next_shift from the
 // updated row still in registers (the next branch's input norm, without re-reading the row).
-// Coefficients (gate * weight, and next_weight * (1 + next_scale), next_shift) are held per
-// wave as in rms_norm_modulate_kernel.
 // One launch serves up to two groups of rows with their own tensors (the image and text streams
-// of a dual-stream block): workgroups [0, blocks0) take group 0, the rest group 1.
+// of a dual-stream block): workgroups [0, rows0) take group 0, the rest group 1.
 struct GatedGroup {
   float* residual;
   const void* branch;
@@ -126,7 +188,7 @@ struct GatedGroup {
 };
 struct GatedArgs {
   GatedGroup g[2];
-  long blocks0;
+  long rows0;
   int width;
   float eps;
 };
@@ -141,7 +203,8 @@ struct GatedArgs {
 template <int NC, typename TB, typename TO, bool SHARED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SHARED && NC == 5 && sizeof(TB) == 2 ? 5 : 1)))
 void gated_residual_kernel(GatedArgs a) {
-  const bool second = blockIdx.x >= a.blocks0;
+  const long blocks0 = (a.rows0 + 3) / 4;
+  const bool second = blockIdx.x >= blocks0;
   const GatedGroup& gg = second ? a.g[1] : a.g[0];
   float* __restrict__ residual = gg.residual;
   const TB* __restrict__ branch = static_cast<const TB*>(gg.branch);
@@ -155,7 +218,7 @@ void gated_residual_kernel(GatedArgs a) {
   TO* __restrict__ next_out = static_cast<TO*>(gg.next_out);
   const int width = a.width;
   const float eps = a.eps;
-  const long row0 = (static_cast<long>(blockIdx.x) - (second ? a.blocks0 : 0)) * 4;
+  const long row0 = (static_cast<long>(blockIdx.x) - (second ? blocks0 : 0)) * 4;
   const long row = row0 + (threadIdx.x >> 6);
   if (!SHARED && row >= rows) return;
   const bool active = row < rows;  // (SHARED: every wave takes part in the LDS fill)
@@ -189,13 +252,12 @@ void gated_residual_kernel(GatedArgs a) {
   }
   float ss = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int j = lane + i * kWave;
-    if (j < nc)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += v[i][e] * v[i][e];
-  }
-  const float r = rsqrtf(wave_sum(ss) / static_cast<float>(width) + eps);
+  for (int i = 0; i < NC; ++i)
+    if (lane + i * kWave < nc) {
+      ss += chunk_sq(v[i]);
+      v[i].reread();
+    }
+  const float r = rms_scale(wave_sum(ss), width, eps);
   const long b = row / rows_per_batch;
   float ss2 = 0.0f;
 #pragma unroll
@@ -213,15 +275,13 @@ void gated_residual_kernel(GatedArgs a) {
         for (int e = 0; e < 8; ++e) gw[e] = g[e] * w[e];
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[i][e] += gw[e] * (v[i][e] * r);
-        ss2 += x[i][e] * x[i][e];
-      }
+      for (int e = 0; e < 8; ++e) x[i][e] = __builtin_fmaf(gw[e], v[i][e] * r, x[i][e]);
+      ss2 += chunk_sq(x[i]);
       store8(res + 8 * j, x[i]);
     }
   }
   if (next_out == nullptr) return;
-  const float r2 = rsqrtf(wave_sum(ss2) / static_cast<float>(width) + eps);
+  const float r2 = rms_scale(wave_sum(ss2), width, eps);
   TO* o = next_out + row * width;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
@@ -240,10 +300,51 @@ void gated_residual_kernel(GatedArgs a) {
         for (int e = 0; e < 8; ++e) m[e] = w2[e] * (1.0f + s1[e]);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = (x[i][e] * r2) * m[e] + c0[e];
+      for (int e = 0; e < 8; ++e) y[e] = __builtin_fmaf(x[i][e] * r2, m[e], c0[e]);
       store8(o + 8 * j, y);
     }
   }
+}
+
+// The split form for few rows: a workgroup of NC waves per row, one 8-element chunk per thread; every
+// load of the row, coefficients included, is in flight before its first reduction (latency bounds it).
+template <int NC, typename TB, typename TO>
+__global__ __launch_bounds__(64 * NC) void gated_residual_split_kernel(GatedArgs a) {
+  __shared__ float part[2][NC][kWave];
+  const bool second = blockIdx.x >= a.rows0;
+  const GatedGroup& gg = second ? a.g[1] : a.g[0];
+  const long row = static_cast<long>(blockIdx.x) - (second ? a.rows0 : 0);
+  const int lane = threadIdx.x & 63, i = threadIdx.x >> 6, j = threadIdx.x;
+  const int width = a.width;
+  const bool in = j < width >> 3, next = gg.next_out != nullptr;
+  const long b = row / gg.rows_per_batch;
+  float* __restrict__ res = gg.residual + row * width + 8 * j;
+  Chunk8<TB> v;
+  float x[8], w[8], g[8], w2[8], s1[8], c0[8];
+  if (in) {
+    v.load(static_cast<const TB*>(gg.branch) + row * width + 8 * j);
+    load8(res, x);
+    load8(gg.weight + 8 * j, w);
+    load8(gg.gate + b * gg.mod_stride + 8 * j, g);
+    if (next) {
+      load8(gg.next_weight + 8 * j, w2);
+      load8(gg.next_scale + b * gg.next_mod_stride + 8 * j, s1);
+      load8(gg.next_shift + b * gg.next_mod_stride + 8 * j, c0);
+    }
+  }
+  const float r = rms_scale(split_row_sum<NC>(in ? chunk_sq(v) : 0.0f, part[0], i, lane), width, a.eps);
+  if (in) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = __builtin_fmaf(g[e] * w[e], v[e] * r, x[e]);
+    store8(res, x);
+  }
+  if (!next) return;
+  const float r2 = rms_scale(split_row_sum<NC>(in ? chunk_sq(x) : 0.0f, part[1], i, lane), width, a.eps);
+  if (!in) return;
+  float y[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) y[e] = __builtin_fmaf(x[e] * r2, w2[e] * (1.0f + s1[e]), c0[e]);
+  store8(static_cast<TO*>(gg.next_out) + row * width + 8 * j, y);
 }
 
 // 16 lanes per (token, head) row of 128 values; lane s owns elements [8s, 8s+8) = rotary
@@ -420,54 +521,53 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(const float* __restrict_
 // out[r] = rmsnorm(residual[r]) * weight (+ add_rows[r % add_period]): the pre-norm residual
 // step of the text adapter's blocks, fused with the next input norm, or its final norm plus
 // the position table.
+// A workgroup of NC waves per row, one chunk per thread, as gated_residual_split_kernel; us per call at
+// width 2560, BF16 in and out, from HBM, against a wave per row: 333 rows 8.3 -> 4.8, 1280: 12.2 ->
+// 10.3, 3600: 26.2 -> 23.9, 8704: 59.5 -> 51.9.
 template <int NC, typename TB, typename TO>
-__global__ __launch_bounds__(256) void residual_norm_kernel(float* __restrict__ residual, const TB* __restrict__ branch,
-                                                            const float* __restrict__ weight,
-                                                            const float* __restrict__ add_rows, long add_period,
-                                                            long rows, int width, float eps, TO* __restrict__ out) {
-  const long row = static_cast<long>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
-  const int lane = threadIdx.x & 63;
-  const int nc = width >> 3;
-  float* res = residual + row * width;
-  float x[NC][8];
-  float ss = 0.0f;
+__global__ __launch_bounds__(64 * NC) void residual_norm_kernel(float* __restrict__ residual,
+                                                                      const TB* __restrict__ branch,
+                                                                      const float* __restrict__ weight,
+                                                                      const float* __restrict__ add_rows,
+                                                                      long add_period, int width, float eps,
+                                                                      TO* __restrict__ out) {
+  __shared__ float part[NC][kWave];
+  const long row = blockIdx.x;
+  const int lane = threadIdx.x & 63, i = threadIdx.x >> 6, j = threadIdx.x;
+  const bool in = j < width >> 3;
+  float* __restrict__ res = residual + row * width + 8 * j;
+  float x[8], w[8], a[8];
+  if (in) {
+    load8(res, x);
+    load8(weight + 8 * j, w);
+    if (add_rows) load8(add_rows + (row % add_period) * width + 8 * j, a);
+    if (branch) {
+      float v[8];
+      load8(branch + row * width + 8 * j, v);
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int j = lane + i * kWave;
-    if (j < nc) {
-      load8(res + 8 * j, x[i]);
-      if (branch) {
-        float v[8];
-        load8(branch + row * width + 8 * j, v);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[i][e] += v[e];
-        store8(res + 8 * j, x[i]);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += x[i][e] * x[i][e];
+      for (int e = 0; e < 8; ++e) x[e] += v[e];
+      store8(res, x);
     }
   }
-  const float r = rsqrtf(wave_sum(ss) / static_cast<float>(width) + eps);
-  TO* o = out + row * width;
-  const float* add = add_rows ? add_rows + (row % add_period) * width : nullptr;
+  const float r = rms_scale(split_row_sum<NC>(in ? chunk_sq(x) : 0.0f, part, i, lane), width, eps);
+  if (!in) return;
+  float y[8];
 #pragma unroll
-  for (int i = 0; i < NC; ++i) {
-    const int j = lane + i * kWave;
-    if (j < nc) {
-      float w[8], y[8];
-      load8(weight + 8 * j, w);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = (x[i][e] * r) * w[e];
-      if (add) {
-        float a[8];
-        load8(add + 8 * j, a);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] += a[e];
-      }
-      store8(o + 8 * j, y);
-    }
-  }
+  for (int e = 0; e < 8; ++e) y[e] = add_rows ? __builtin_fmaf(x[e] * r, w[e], a[e]) : (x[e] * r) * w[e];
+  store8(out + row * width + 8 * j, y);
+}
+
+// f(TI{}, TO{}) of the C++ types of two dtype codes.
+template <typename F>
+void with_types(int in_dtype, int out_dtype, F&& f) {
+  if (in_dtype == IRIS_F32 && out_dtype == IRIS_BF16)
+    f(float{}, bf16{});
+  else if (in_dtype == IRIS_F32)
+    f(float{}, float{});
+  else if (out_dtype == IRIS_BF16)
+    f(bf16{}, bf16{});
+  else
+    f(bf16{}, float{});
 }
 
 template <int NC, bool SHARED>
@@ -544,33 +644,40 @@ int gated_launch(int groups, const GatedGroup* g, int branch_dtype, int width, f
   IRIS_REQUIRE(width > 0 && width % 128 == 0 && width <= 8192,
                "gated_residual_rms_norm_ shape mismatch: width %% 128 == 0 and <= 8192 (got %d)", width);
   GatedArgs a{};
-  long blocks = 0;
+  long rows = 0;
   for (int i = 0; i < groups; ++i) {
     const int rc = check_group(g[i]);
     if (rc) return rc;
     IRIS_REQUIRE((g[i].next_out == nullptr) == (g[0].next_out == nullptr),
                  "gated_residual_rms_norm: both groups with or both without the next norm");
     a.g[i] = g[i];
-    const long b = (g[i].rows + kRowsPerBlock - 1) / kRowsPerBlock;
-    if (i == 0) a.blocks0 = b;
-    blocks += b;
+    rows += g[i].rows;
   }
   if (groups == 1) a.g[1] = a.g[0];
+  a.rows0 = g[0].rows;
   a.width = width;
   a.eps = eps;
-  if (blocks == 0) return IRIS_OK;
-  IRIS_REQUIRE(blocks < (1L << 31), "gated_residual_rms_norm: too many rows");
-  const dim3 grid(static_cast<unsigned>(blocks));
-  // with the next norm, coefficients in LDS when every workgroup's four rows share a batch
-  // index (without it the LDS fill and its barrier cost more than the one coefficient row saves)
-  const bool next = g[0].next_out != nullptr;
-  bool shared = next && 3L * width * sizeof(float) <= 48 * 1024;
-  for (int i = 0; i < groups; ++i) shared = shared && g[i].rows_per_batch % kRowsPerBlock == 0;
+  if (rows == 0) return IRIS_OK;
+  IRIS_REQUIRE(rows < (1L << 31), "gated_residual_rms_norm: too many rows");
+  if (rows > kGatedSplitRows) {
+    const dim3 grid(static_cast<unsigned>((a.rows0 + 3) / 4 + (groups > 1 ? (g[1].rows + 3) / 4 : 0)));
+    // with the next norm, coefficients in LDS when every workgroup's four rows share a batch
+    // index (without it the LDS fill and its barrier cost more than the one coefficient row saves)
+    bool shared = g[0].next_out != nullptr && 3L * width * sizeof(float) <= 48 * 1024;
+    for (int i = 0; i < groups; ++i) shared = shared && g[i].rows_per_batch % kRowsPerBlock == 0;
+    IRIS_NC_DISPATCH(nc_bucket(width), {
+      if (branch_dtype == IRIS_BF16)
+        launch_gated<NC, bf16>(grid, stream, a, out_dtype, shared);
+      else
+        launch_gated<NC, float>(grid, stream, a, out_dtype, shared);
+    })
+    return check_launch("gated_residual_rms_norm");
+  }
+  const dim3 grid(static_cast<unsigned>(rows));
   IRIS_NC_DISPATCH(nc_bucket(width), {
-    if (branch_dtype == IRIS_BF16)
-      launch_gated<NC, bf16>(grid, stream, a, out_dtype, shared);
-    else
-      launch_gated<NC, float>(grid, stream, a, out_dtype, shared);
+    with_types(branch_dtype, out_dtype, [&](auto tb, auto to) {
+      gated_residual_split_kernel<NC, decltype(tb), decltype(to)><<<grid, 64 * NC, 0, stream>>>(a);
+    });
   })
   return check_launch("gated_residual_rms_norm");
 }
@@ -599,6 +706,18 @@ extern "C" int iris_rms_norm_modulate(const void* x, int x_dtype, void* out, int
                "rms_norm_modulate: modulation rows must be 16-byte aligned (mod_stride %% 4 == 0)");
   IRIS_REQUIRE(x && out && weight && shift && scale, "rms_norm_modulate: null pointer");
   if (rows == 0) return IRIS_OK;
+  if (rows <= modulate_split_rows(x_dtype)) {
+    IRIS_NC_DISPATCH(nc_bucket(width), {
+      with_types(x_dtype, out_dtype, [&](auto ti, auto to) {
+        using TI = decltype(ti);
+        using TO = decltype(to);
+        rms_norm_modulate_split_kernel<NC, TI, TO><<<dim3(static_cast<unsigned>(rows)), 64 * NC, 0, stream>>>(
+            static_cast<const TI*>(x), static_cast<TO*>(out), weight, shift, scale, rows_per_batch, width, mod_stride,
+            eps);
+      });
+    })
+    return check_launch("rms_norm_modulate");
+  }
   const dim3 grid(static_cast<unsigned>((rows + kRowsPerBlock - 1) / kRowsPerBlock));
   // coefficients in LDS when every workgroup's four rows share a batch index
   const bool shared = rows_per_batch % kRowsPerBlock == 0 && 2L * width * sizeof(float) <= 32 * 1024;
@@ -778,22 +897,14 @@ extern "C" int iris_residual_rms_norm(float* residual, const void* branch, int b
   IRIS_REQUIRE(out != residual && (!branch || (branch != residual && branch != out)),
                "residual_rms_norm: out and branch must not alias the residual");
   if (rows == 0) return IRIS_OK;
-  const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
+  IRIS_REQUIRE(rows < (1L << 31), "residual_rms_norm: too many rows");
   IRIS_NC_DISPATCH(nc_bucket(width), {
-    if (branch_dtype == IRIS_BF16 && out_dtype == IRIS_BF16)
-      residual_norm_kernel<NC, bf16, bf16><<<grid, 256, 0, stream>>>(residual, (const bf16*)branch, weight, add_rows,
-                                                                     add_period, rows, width, eps, (bf16*)out);
-    else if (branch_dtype == IRIS_BF16)
-      residual_norm_kernel<NC, bf16, float><<<grid, 256, 0, stream>>>(residual, (const bf16*)branch, weight, add_rows,
-                                                                      add_period, rows, width, eps, (float*)out);
-    else if (out_dtype == IRIS_BF16)
-      residual_norm_kernel<NC, float, bf16><<<grid, 256, 0, stream>>>(residual, (const float*)branch, weight,
-                                                                      add_rows, add_period, rows, width, eps,
-                                                                      (bf16*)out);
-    else
-      residual_norm_kernel<NC, float, float><<<grid, 256, 0, stream>>>(residual, (const float*)branch, weight,
-                                                                       add_rows, add_period, rows, width, eps,
-                                                                       (float*)out);
+    with_types(branch_dtype, out_dtype, [&](auto tb, auto to) {
+      using TB = decltype(tb);
+      using TO = decltype(to);
+      residual_norm_kernel<NC, TB, TO><<<dim3(static_cast<unsigned>(rows)), 64 * NC, 0, stream>>>(
+          residual, static_cast<const TB*>(branch), weight, add_rows, add_period, width, eps, static_cast<TO*>(out));
+    });
   })
   return check_launch("residual_rms_norm");
 }
