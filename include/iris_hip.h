@@ -215,6 +215,15 @@ int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const void* const* 
                            const float* cos_table, const float* sin_table, long table_rows, void* q, void* k_out,
                            int heads, int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream);
 
+/* iris_gemm_bf16_qk_rope with vt for batch items of any row count and offset: the V heads always reach
+ * vt as iris_v_heads_t writes them, from the store itself where the tile allows it, else from c (whose V
+ * columns may or may not be written). Same arguments; vt is required. */
+int iris_gemm_bf16_qkv(int groups, const void* const* a, const void* const* b, void* const* c, const int* m, int n,
+                       int k, long lda, long ldb, long ldc, const float* const* q_weight, const float* const* k_weight,
+                       const int* rows_per_batch, const int* dst_offset, const float* cos_table,
+                       const float* sin_table, long table_rows, void* q, void* k_out, int heads, int kv_heads,
+                       long n_dst, void* vt, long n_vt, float eps, hipStream_t stream);
+
 /* Matrix-vector products for the timestep MLP and the shared adaLN cores
  * (src/iris_metal/model.py:190-192; src/iris3b/nn/modulation.py:258-285):
  * y[b, n] = act_out(sum_k W[n, k] act_in(x[b, k]) + bias[n]), W BF16 [n, k];

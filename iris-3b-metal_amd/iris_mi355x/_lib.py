@@ -47,6 +47,8 @@ _SIGNATURES: dict[str, list] = {
     "iris_gemm_bf16_grouped": [c_int, P, P, P, P, P, c_int, c_int, c_int, c_long, c_long, c_long, c_int, P],
     "iris_gemm_bf16_qk_rope": [c_int, P, P, P, P, c_int, c_int, c_long, c_long, c_long, P, P, P, P, P, P, c_long,
                                P, P, c_int, c_int, c_long, P, c_long, c_float, P],
+    "iris_gemm_bf16_qkv": [c_int, P, P, P, P, c_int, c_int, c_long, c_long, c_long, P, P, P, P, P, P, c_long,
+                               P, P, c_int, c_int, c_long, P, c_long, c_float, P],
     "iris_gemv_bf16": [P, P, c_int, c_int, c_int, P, P, c_int, P, c_int, c_int, P],
     "iris_gemv_bf16_pair": [P, P, c_int, P, c_int, P, P, P, P, c_int, c_int, P],
     "iris_timestep_gemv_bf16": [P, P, c_int, P, c_int, c_int, P, P, c_int, P],

@@ -270,8 +270,8 @@ __device__ __forceinline__ void qk_store(bf16* cl, const TileJob& job, int N, lo
 // kEpiQkRope on 128-wide tiles (one head, or 128 plain columns, per tile), once the BF16 tile is
 // staged in LDS (16-byte chunk c of row r at c ^ (r & 15)): 16 lanes per row, one chunk each, so a
 // head is normed and rotated by head_norm_rope in registers and leaves as whole 256-byte rows; the
-// V heads transposed per 16-position group (rows_per_batch and dst_offset are multiples of 16 with
-// vt, so a group lies inside one batch item); the other columns to C.
+// V heads with vt transposed, per 16-position group where rows_per_batch and dst_offset are multiples
+// of 16 (a group then lies inside one batch item), else token by token; the other columns to C.
 template <int BM, int NW>
 __device__ __forceinline__ void qk_store_head(const bf16* cl, const TileJob& job, long ldc, const QkRope& qk) {
   constexpr int OUT_N = 128;
@@ -303,6 +303,27 @@ __device__ __forceinline__ void qk_store_head(const bf16* cl, const TileJob& job
       for (int e = 0; e < 8; ++e) a[e] = to_f32(v[e]);
       head_norm_rope(a, wg, cs, sn, qk.eps, y);
       if (m0 + r < M) store8(dst + ((static_cast<long>(b) * heads + head) * qk.n_dst + pos) * 128 + 8 * c, y);
+    }
+    return;
+  }
+  if (qk.vt && n0 < nqkv && (rpb % 16 || dst_offset % 16)) {
+    // ragged items: a thread holds 8 dims of one row's token and stores them one by one, a wave's lanes
+    // on 64 consecutive tokens of a dim (two bytes each, within 16-position groups in slot order)
+    const int vh = (n0 - nqk) >> 7;
+    const int lane = tid & 63;
+#pragma unroll 1
+    for (int r = lane; r < (BM + 63) / 64 * 64; r += 64) {
+      const int m = m0 + r;
+      if (r >= BM || m >= M) continue;
+      const int b = m / rpb;
+      const int pos = vt_slot(dst_offset + (m - b * rpb));
+      bf16* vtp = qk.vt + (static_cast<long>(b) * qk.kv_heads + vh) * 128 * static_cast<long>(qk.n_vt) + pos;
+#pragma unroll 1
+      for (int ch = tid >> 6; ch < 16; ch += NW) {
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(cl + r * OUT_N + 8 * (ch ^ (r & 15)));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vtp[static_cast<long>(8 * ch + e) * qk.n_vt] = v[e];
+      }
     }
     return;
   }
@@ -2001,7 +2022,7 @@ extern "C" int iris_gemm_bf16_grouped(int groups, const void* const* a, const vo
   return launch_two(a1, plan.tile1, epilogue, a2, plan.tile2, epilogue, c_dtype, stream);
 }
 
-extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const void* const* b, void* const* c,
+static int qk_rope_gemm(bool any_rows, int groups, const void* const* a, const void* const* b, void* const* c,
                                       const int* m, int n, int k, long lda, long ldb, long ldc,
                                       const float* const* q_weight, const float* const* k_weight,
                                       const int* rows_per_batch, const int* dst_offset, const float* cos_table,
@@ -2043,6 +2064,10 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
     IRIS_REQUIRE(aligned(vt, 16) && n_vt > 0 && n_vt % 64 == 0 && n_vt < (1L << 30),
                  "gemm_qk_rope: vt must be 16-byte aligned with n_vt a positive multiple of 64");
     for (int i = 0; i < groups; ++i)
+      IRIS_REQUIRE(!any_rows || m[i] == 0 || dst_offset[i] + static_cast<long>(rows_per_batch[i]) <= n_vt,
+                   "gemm_qkv: positions outside vt (group %d: %d rows at %d, n_vt %ld)", i, rows_per_batch[i],
+                   dst_offset[i], n_vt);
+    for (int i = 0; i < groups && !any_rows; ++i)
       IRIS_REQUIRE(m[i] == 0 || (rows_per_batch[i] % 256 == 0 && dst_offset[i] % 16 == 0 &&
                                  dst_offset[i] + static_cast<long>(rows_per_batch[i]) <= n_vt),
                    "gemm_qk_rope: the V^T store needs rows_per_batch %% 256 == 0, dst_offset %% 16 == 0 and "
@@ -2091,6 +2116,23 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
   }
   if (ring >= 0)
     return gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, ring, stream, &qk);
+  // the 256 x 256 store transposes whole 256-row items only: otherwise the V columns go to c and from
+  // there to vt in a launch of their own
+  bool whole = true;
+  for (int i = 0; i < groups; ++i) whole = whole && rows_per_batch[i] % 256 == 0 && dst_offset[i] % 16 == 0;
+  if (vt && !whole) {
+    const int rc = qk_rope_gemm(false, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch,
+                                dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, nullptr,
+                                0, eps, stream);
+    if (rc != IRIS_OK) return rc;
+    for (int i = 0; i < groups; ++i) {
+      const int vrc = m[i] == 0 ? IRIS_OK
+                                : iris_v_heads_t(c[i], vt, m[i] / rows_per_batch[i], rows_per_batch[i], n_vt, kv_heads,
+                                                 dst_offset[i], ldc, (heads + kv_heads) * 128L, stream);
+      if (vrc != IRIS_OK) return vrc;
+    }
+    return IRIS_OK;
+  }
   if (n <= n_qkv)
     return gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, kQkRopeTile, stream, &qk);
   // the columns after the V heads (the gate columns of a q | k | v | gate weight) are a plain
@@ -2107,6 +2149,26 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
   rc = make_args(a2, groups, a, b2, nullptr, c2, m, n - n_qkv, k, lda, ldb, ldc, IRIS_EPI_NONE, tile2, nullptr);
   if (rc != IRIS_OK) return rc;
   return launch_two(a1, kQkRopeTile, kEpiQkRope, a2, tile2, IRIS_EPI_NONE, IRIS_BF16, stream);
+}
+
+// (with vt, iris_gemm_bf16_qk_rope takes whole 256-row items only, iris_gemm_bf16_qkv any)
+extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const void* const* b, void* const* c,
+                                      const int* m, int n, int k, long lda, long ldb, long ldc,
+                                      const float* const* q_weight, const float* const* k_weight,
+                                      const int* rows_per_batch, const int* dst_offset, const float* cos_table,
+                                      const float* sin_table, long table_rows, void* q, void* k_out, int heads,
+                                      int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream) {
+  return qk_rope_gemm(false, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch, dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, vt, n_vt, eps, stream);
+}
+
+extern "C" int iris_gemm_bf16_qkv(int groups, const void* const* a, const void* const* b, void* const* c,
+                                      const int* m, int n, int k, long lda, long ldb, long ldc,
+                                      const float* const* q_weight, const float* const* k_weight,
+                                      const int* rows_per_batch, const int* dst_offset, const float* cos_table,
+                                      const float* sin_table, long table_rows, void* q, void* k_out, int heads,
+                                      int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream) {
+  IRIS_REQUIRE(vt, "gemm_qkv: null vt");
+  return qk_rope_gemm(true, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch, dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, vt, n_vt, eps, stream);
 }
 
 extern "C" int iris_gemm_bf16(const void* a, const void* b, const float* bias, void* c, int c_dtype, int m, int n,

@@ -16,8 +16,8 @@ Data layout in HBM (per call shape, allocated once and reused):
   batch item ``Y`` and ``X`` are its first ``T`` and last ``L`` rows, so the join copies nothing);
 - packed projections ``[rows, 6400]`` = ``q | k | v | gate``: one call per block over the packed
   weight (two GEMMs in one launch), the q | k | v one writing the attention inputs below
-  straight from its store (Q / K normed and rotated; V transposed when each batch item is whole
-  256-row tiles, else its V columns land here for ``v_heads_t``), the gate one its columns here;
+  straight from its store (Q / K normed and rotated, V transposed; on the 256 x 256 store ragged
+  items' V columns land here first), the gate one its columns here;
 - attention inputs ``q`` ``[B, 20, N_pad, 128]``, ``k`` ``[B, 5, N_pad, 128]``, ``v^T`` ``[B, 5, 128, N_pad]``;
 - pixel stream ``[B*L, p*p, 16]`` FP32 and its BF16 normed copy, adaLN mods ``[B*L, p*p, 64]`` BF16.
 """
@@ -499,7 +499,6 @@ class HipIris:
         X, Y = ws["X"].view(B, Lp, D), ws["Y"].view(B, T, D)
         xm = [self._mods(ws, "mods_img", blk["img_mod"], c) for c in range(6)]
         ym = [self._mods(ws, "mods_txt", blk["txt_mod"], c) for c in range(6)]
-        qkvg_w = ws["qkvg"].shape[1]
         rows_x, rows_y = B * Lp, B * T
         hx, hy = ws["h_tok"][:rows_x], ws["h_tok"][rows_x:rows_x + rows_y]
         px, py = ws["qkvg"][:rows_x], ws["qkvg"][rows_x:rows_x + rows_y]
@@ -512,18 +511,14 @@ class HipIris:
             K.rms_norm_modulate(X, blk["norm_x1"], xm[0], xm[1], eps, bf16, out=hx.view(B, Lp, D))
             K.rms_norm_modulate(Y, blk["norm_y1"], ym[0], ym[1], eps, bf16, out=hy.view(B, T, D))
         # q | k | v | gate in one launch, the Q / K norm + rotary in the store of the q | k | v
-        # columns (text rows at positions 0.., image rows after them), the V heads transposed
-        # there too or from its output, the gate columns a plain product beside them
+        # columns (text rows at positions 0.., image rows after them), the V heads transposed,
+        # the gate columns a plain product beside them
         rope_c, rope_s = ws["rope"]
         q, k, vt = ws["q"], ws["k"], ws["vt"]
         gate_col = (H + 2 * Hkv) * HEAD_DIM
-        fuse_vt = Lp % 256 == 0 and T % 256 == 0  # whole 256-row tiles per item (and T % 16 == 0)
         K.linear_qk_rope([hx, hy], [blk["qkvg_x"], blk["qkvg_y"]], [px, py], [blk["q_norm_x"], blk["q_norm_y"]],
                          [blk["k_norm_x"], blk["k_norm_y"]], rope_c, rope_s, eps, H, Hkv, q, k, [Lp, T], [T, 0],
-                         vt=vt if fuse_vt else None)
-        if not fuse_vt:
-            for proj, rows, off in ((py, T, 0), (px, Lp, T)):
-                K.v_heads_t(proj.view(B, rows, qkvg_w), Hkv, vt, (H + Hkv) * HEAD_DIM, off)
+                         vt=vt, any_rows=True)
         K.flash_attention(q, k, vt, N, ay, ax, n_split=T, gate0=py[:, gate_col:], gate1=px[:, gate_col:])
         K.linear_grouped([ax, ay], [blk["proj_x_w"], blk["proj_y_w"]], [blk["proj_x_b"], blk["proj_y_b"]], [bx, by])
         K.gated_residual_grouped_([X, Y], [bx.view(B, Lp, D), by.view(B, T, D)],
@@ -553,17 +548,13 @@ class HipIris:
         m = [self._mods(ws, "mods_img", blk["img_mod"], c) for c in range(6)]
         rows = B * N
         h, proj = ws["h_tok"][:rows], ws["qkvg"][:rows]
-        qkvg_w = proj.shape[1]
         if not h_ready:
             K.rms_norm_modulate(tok.view(B, N, D), blk["norm1"], m[0], m[1], eps, torch.bfloat16, out=h.view(B, N, D))
         rope_c, rope_s = ws["rope"]
         q, k, vt = ws["q"], ws["k"], ws["vt"]
         gate_col = (H + 2 * Hkv) * HEAD_DIM  # as in _dual_block
-        fuse_vt = N % 256 == 0
         K.linear_qk_rope([h], [blk["qkvg"]], [proj], [blk["q_norm"]], [blk["k_norm"]],
-                         rope_c, rope_s, eps, H, Hkv, q, k, [N], [0], vt=vt if fuse_vt else None)
-        if not fuse_vt:
-            K.v_heads_t(proj.view(B, N, qkvg_w), Hkv, vt, (H + Hkv) * HEAD_DIM)
+                         rope_c, rope_s, eps, H, Hkv, q, k, [N], [0], vt=vt, any_rows=True)
         gate = proj[:, gate_col:]
         if not last:
             R, M, per_batch = tok, rows, N

@@ -74,12 +74,12 @@ def test_ring_two_groups(tile, rows):
 
 
 @pytest.mark.parametrize("tile", [t for t, (_, bn, _) in RING.items() if bn == 128])
-@pytest.mark.parametrize("heads,kv_heads,tokens,batch,gate", [(3, 1, (37,), 2, True), (2, 2, (60, 77), 1, False),
+@pytest.mark.parametrize("heads,kv_heads,tokens,batch,gate", [(3, 1, (37,), 2, True), (2, 2, (60, 77), 1, False), (2, 1, (48, 80), 2, True),
                                                              (4, 2, (256,), 2, True), (2, 1, (256, 256), 1, True)])
 def test_ring_qk_store(tile, heads, kv_heads, tokens, batch, gate):
     """The q | k | v (| gate) store on ring tiles writes what the plain product followed by
-    qkv_prepare writes and nothing else: ragged batch items, two streams, and with whole 256-row
-    items the V heads transposed too."""
+    qkv_prepare writes and nothing else: whole and ragged batch items and offsets, two streams, the V
+    heads plain or transposed."""
     g = torch.Generator(device=DEV).manual_seed(43)
     n_qkv = (heads + 2 * kv_heads) * 128
     n = n_qkv + (128 * heads if gate else 0)
@@ -99,16 +99,40 @@ def test_ring_qk_store(tile, heads, kv_heads, tokens, batch, gate):
     for out, qw, kw, t, off in zip(plain, *gains, tokens, offsets):
         K.qkv_prepare(out.view(batch, t, n), qw, kw, cos, sin, 1e-6, heads, kv_heads, q_ref, k_ref, vt_ref, 0,
                       heads * 128, v_col, off)
-    for with_vt in (False, True) if all(t % 256 == 0 for t in tokens) else (False,):
+    for with_vt in (False, True):
         q, key, vt = buffers()
         outs = [torch.full((batch * t, n), 5.0, device=DEV, dtype=torch.bfloat16) for t in tokens]
         forced(tile, lambda: K.linear_qk_rope(xs, ws, outs, *gains, cos, sin, 1e-6, heads, kv_heads, q, key,
-                                              list(tokens), offsets, vt=vt if with_vt else None))
+                                              list(tokens), offsets, vt=vt if with_vt else None, any_rows=True))
         assert torch.equal(q, q_ref) and torch.equal(key, k_ref)
         assert torch.equal(vt, vt_ref) if with_vt else torch.all(vt == 3.0)
         first = n_qkv if with_vt else v_col
         for out, ref in zip(outs, plain):
             assert torch.equal(out[:, first:], ref[:, first:]) and torch.all(out[:, :first] == 5.0)
+
+
+@pytest.mark.parametrize("tokens,batch", [((300, 77), 1), ((272,), 2), ((256, 512), 1)])
+def test_qkv_of_any_rows_without_ring_tiles(tokens, batch):
+    """On the 256 x 256 store ragged items reach the V^T layout through the output's V columns."""
+    g = torch.Generator(device=DEV).manual_seed(45)
+    heads, kv_heads, k = 2, 1, 256
+    n, v_col = 6 * 128, 3 * 128
+    offsets = [tokens[1], 0] if len(tokens) == 2 else [0]
+    n_pad = (sum(tokens) + 63) // 64 * 64
+    cos, sin = (torch.randn(n_pad, 64, generator=g, device=DEV) for _ in range(2))
+    xs, ws = [randn(g, batch * t, k) for t in tokens], [randn(g, n, k, scale=0.05) for _ in tokens]
+    gains = [[torch.ones(128, device=DEV) for _ in tokens] for _ in range(2)]
+    bufs = [[torch.full((batch, h, *s), 3.0, device=DEV, dtype=torch.bfloat16)
+             for h, s in ((heads, (n_pad, 128)), (kv_heads, (n_pad, 128)), (kv_heads, (128, n_pad)))] for _ in range(2)]
+    outs = [torch.empty(batch * t, n, device=DEV, dtype=torch.bfloat16) for t in tokens]
+    for x, w, qw, kw, t, off in zip(xs, ws, *gains, tokens, offsets):
+        plain = forced(16, lambda x=x, w=w: K.linear(x, w))
+        K.qkv_prepare(plain.view(batch, t, n), qw, kw, cos, sin, 1e-6, heads, kv_heads, *bufs[0], 0, heads * 128, v_col,
+                      off)
+    forced(16, lambda: K.linear_qk_rope(xs, ws, outs, *gains, cos, sin, 1e-6, heads, kv_heads, *bufs[1][:2],
+                                        list(tokens), offsets, vt=bufs[1][2], any_rows=True))
+    for got, want in zip(bufs[1], bufs[0]):
+        assert torch.equal(got, want)
 
 
 def test_ring_refuses_a_k_loop_shorter_than_its_ring():
