@@ -58,6 +58,20 @@ int iris_gated_residual_norm_modulate(float* residual, const void* branch, int b
                                       const float* next_scale, long next_mod_stride, void* next_out,
                                       int next_out_dtype, hipStream_t stream);
 
+/* iris_rms_norm_modulate of FP32 rows that also enter a residual stream: row r of batch item b goes,
+ * normed and modulated, to row b dst_batch_rows + dst_offset + r of out and, as it is, of copy. */
+int iris_rms_norm_modulate_copy(const float* x, void* out, int out_dtype, float* copy, const float* weight,
+                                const float* shift, const float* scale, long rows, long rows_per_batch, int width,
+                                long mod_stride, float eps, long dst_batch_rows, long dst_offset, hipStream_t stream);
+
+/* iris_gated_residual_rms_norm of one or two streams that also leave it: of each batch item the first
+ * split[i] updated rows are written to copy0[i] as well (packed), the rest to copy1[i]. Arrays as in
+ * iris_gated_residual_grouped. */
+int iris_gated_residual_copy(int groups, float* const* residual, const void* const* branch, int branch_dtype,
+                             const float* const* weight, const float* const* gate, const long* rows,
+                             const long* rows_per_batch, int width, const long* mod_stride, float eps,
+                             float* const* copy0, float* const* copy1, const long* split, hipStream_t stream);
+
 /* The image- and text-stream calls of a dual-stream block in one launch (no reference
  * counterpart; the reference calls gated_residual_rms_norm_ once per stream,
  * model.py:286-289, 311-313): group i is iris_gated_residual_rms_norm (next_out == NULL) or

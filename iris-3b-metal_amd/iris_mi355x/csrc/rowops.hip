@@ -140,14 +140,17 @@ __global__ __launch_bounds__(256) void rms_norm_modulate_kernel(const TI* __rest
   }
 }
 
-// rms_norm_modulate_kernel with a workgroup of NC waves per row, one chunk per thread.
+// rms_norm_modulate_kernel with a workgroup of NC waves per row, one chunk per thread. Row r of batch
+// item b goes to row b dst_batch_rows + dst_offset + r of out, and unchanged to that row of `copy`
+// where one is given (a block's input entering the residual stream).
 template <int NC, typename TI, typename TO>
 __global__ __launch_bounds__(64 * NC) void rms_norm_modulate_split_kernel(const TI* __restrict__ x, TO* __restrict__ out,
                                                                           const float* __restrict__ weight,
                                                                           const float* __restrict__ shift,
                                                                           const float* __restrict__ scale,
                                                                           long rows_per_batch, int width,
-                                                                          long mod_stride, float eps) {
+                                                                          long mod_stride, float eps, float* copy,
+                                                                          long dst_batch_rows, long dst_offset) {
   __shared__ float part[NC][kWave];
   const long row = blockIdx.x;
   const int lane = threadIdx.x & 63, i = threadIdx.x >> 6, j = threadIdx.x;
@@ -161,12 +164,19 @@ __global__ __launch_bounds__(64 * NC) void rms_norm_modulate_split_kernel(const 
     load8(scale + b * mod_stride + 8 * j, s1);
     load8(shift + b * mod_stride + 8 * j, c0);
   }
+  const long dst = (b * dst_batch_rows + dst_offset + (row - b * rows_per_batch)) * width + 8 * j;
+  if (copy && in) {
+    float x8[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x8[e] = v[e];
+    store8(copy + dst, x8);
+  }
   const float r = rms_scale(split_row_sum<NC>(in ? chunk_sq(v) : 0.0f, part, i, lane), width, eps);
   if (!in) return;
   float y[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) y[e] = __builtin_fmaf(v[e] * r, w[e] * (1.0f + s1[e]), c0[e]);
-  store8(out + row * width + 8 * j, y);
+  store8(out + dst, y);
 }
 
 // residual[r] += gate * rmsnorm(branch[r]) * weight; with next_out, also
@@ -185,6 +195,15 @@ struct GatedGroup {
   const float* next_scale;
   long next_mod_stride;
   void* next_out;
+  // the updated rows again (a block's output leaving the residual stream), or null: of each batch item
+  // the first `also_split` rows to also0, the rest to also1, both packed
+  float *also0, *also1;
+  long also_split;
+  __device__ float* also_row(long row, int width) const {
+    const long b = row / rows_per_batch, r = row - b * rows_per_batch;
+    return r < also_split ? also0 + (b * also_split + r) * width
+                          : also1 + (b * (rows_per_batch - also_split) + r - also_split) * width;
+  }
 };
 struct GatedArgs {
   GatedGroup g[2];
@@ -278,6 +297,7 @@ void gated_residual_kernel(GatedArgs a) {
       for (int e = 0; e < 8; ++e) x[i][e] = __builtin_fmaf(gw[e], v[i][e] * r, x[i][e]);
       ss2 += chunk_sq(x[i]);
       store8(res + 8 * j, x[i]);
+      if (!SHARED && gg.also1) store8(gg.also_row(row, width) + 8 * j, x[i]);
     }
   }
   if (next_out == nullptr) return;
@@ -337,6 +357,7 @@ __global__ __launch_bounds__(64 * NC) void gated_residual_split_kernel(GatedArgs
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = __builtin_fmaf(g[e] * w[e], v[e] * r, x[e]);
     store8(res, x);
+    if (gg.also1) store8(gg.also_row(row, width) + 8 * j, x);
   }
   if (!next) return;
   const float r2 = rms_scale(split_row_sum<NC>(in ? chunk_sq(x) : 0.0f, part[1], i, lane), width, a.eps);
@@ -686,7 +707,8 @@ int gated_common(float* residual, const void* branch, int branch_dtype, const fl
                  long rows, long rows_per_batch, int width, long mod_stride, float eps, const float* nw,
                  const float* nsh, const float* nsc, long nstride, void* next_out, int out_dtype,
                  hipStream_t stream) {
-  const GatedGroup g{residual, branch, weight, gate, rows, rows_per_batch, mod_stride, nw, nsh, nsc, nstride, next_out};
+  const GatedGroup g{residual, branch, weight, gate,     rows,    rows_per_batch, mod_stride, nw,
+                     nsh,      nsc,    nstride, next_out, nullptr, nullptr,        0};
   return gated_launch(1, &g, branch_dtype, width, eps, out_dtype, stream);
 }
 
@@ -713,7 +735,7 @@ extern "C" int iris_rms_norm_modulate(const void* x, int x_dtype, void* out, int
         using TO = decltype(to);
         rms_norm_modulate_split_kernel<NC, TI, TO><<<dim3(static_cast<unsigned>(rows)), 64 * NC, 0, stream>>>(
             static_cast<const TI*>(x), static_cast<TO*>(out), weight, shift, scale, rows_per_batch, width, mod_stride,
-            eps);
+            eps, nullptr, rows_per_batch, 0);
       });
     })
     return check_launch("rms_norm_modulate");
@@ -750,6 +772,50 @@ extern "C" int iris_gated_residual_norm_modulate(float* residual, const void* br
                       next_weight, next_shift, next_scale, next_mod_stride, next_out, next_out_dtype, stream);
 }
 
+extern "C" int iris_rms_norm_modulate_copy(const float* x, void* out, int out_dtype, float* copy, const float* weight,
+                                           const float* shift, const float* scale, long rows, long rows_per_batch,
+                                           int width, long mod_stride, float eps, long dst_batch_rows, long dst_offset,
+                                           hipStream_t stream) {
+  IRIS_REQUIRE(valid_dtype(out_dtype), "rms_norm_modulate_copy: unknown dtype");
+  IRIS_REQUIRE(width > 0 && width % 128 == 0 && width <= 8192,
+               "rms_norm_modulate_copy: width %% 128 == 0 and <= 8192 (got %d)", width);
+  IRIS_REQUIRE(rows >= 0 && rows < (1L << 31) && rows_per_batch > 0 && rows % rows_per_batch == 0 && dst_offset >= 0 &&
+                   dst_offset + rows_per_batch <= dst_batch_rows,
+               "rms_norm_modulate_copy: bad row counts");
+  IRIS_REQUIRE(mod_stride % 4 == 0 && aligned(shift, 16) && aligned(scale, 16) && aligned(weight, 16),
+               "rms_norm_modulate_copy: modulation rows must be 16-byte aligned (mod_stride %% 4 == 0)");
+  IRIS_REQUIRE(x && out && copy && weight && shift && scale, "rms_norm_modulate_copy: null pointer");
+  if (rows == 0) return IRIS_OK;
+  IRIS_NC_DISPATCH(nc_bucket(width), {
+    with_types(IRIS_F32, out_dtype, [&](auto, auto to) {
+      using TO = decltype(to);
+      rms_norm_modulate_split_kernel<NC, float, TO><<<dim3(static_cast<unsigned>(rows)), 64 * NC, 0, stream>>>(
+          x, static_cast<TO*>(out), weight, shift, scale, rows_per_batch, width, mod_stride, eps, copy, dst_batch_rows,
+          dst_offset);
+    });
+  })
+  return check_launch("rms_norm_modulate_copy");
+}
+
+extern "C" int iris_gated_residual_copy(int groups, float* const* residual, const void* const* branch, int branch_dtype,
+                                        const float* const* weight, const float* const* gate, const long* rows,
+                                        const long* rows_per_batch, int width, const long* mod_stride, float eps,
+                                        float* const* copy0, float* const* copy1, const long* split,
+                                        hipStream_t stream) {
+  IRIS_REQUIRE(groups == 1 || groups == 2, "gated_residual_copy: 1 or 2 groups");
+  IRIS_REQUIRE(residual && branch && weight && gate && rows && rows_per_batch && mod_stride && copy0 && copy1 && split,
+               "gated_residual_copy: null array");
+  GatedGroup g[2] = {};
+  for (int i = 0; i < groups; ++i) {
+    g[i] = GatedGroup{residual[i], branch[i], weight[i], gate[i], rows[i], rows_per_batch[i], mod_stride[i],
+                      nullptr, nullptr, nullptr, 0, nullptr, copy0[i], copy1[i], split[i]};
+    IRIS_REQUIRE(split[i] >= 0 && split[i] < rows_per_batch[i] && rows[i] % rows_per_batch[i] == 0 && copy1[i] &&
+                     (split[i] == 0 || copy0[i]),
+                 "gated_residual_copy: bad split or copy (group %d)", i);
+  }
+  return gated_launch(groups, g, branch_dtype, width, eps, IRIS_BF16, stream);
+}
+
 extern "C" int iris_gated_residual_grouped(int groups, float* const* residual, const void* const* branch,
                                            int branch_dtype, const float* const* weight, const float* const* gate,
                                            const long* rows, const long* rows_per_batch, int width,
@@ -767,7 +833,7 @@ extern "C" int iris_gated_residual_grouped(int groups, float* const* residual, c
   for (int i = 0; i < groups; ++i) {
     g[i] = GatedGroup{residual[i], branch[i], weight[i], gate[i], rows[i], rows_per_batch[i], mod_stride[i],
                       next ? next_weight[i] : nullptr, next ? next_shift[i] : nullptr, next ? next_scale[i] : nullptr,
-                      next ? next_mod_stride[i] : 0, next ? next_out[i] : nullptr};
+                      next ? next_mod_stride[i] : 0, next ? next_out[i] : nullptr, nullptr, nullptr, 0};
     IRIS_REQUIRE(!next || g[i].next_out, "gated_residual_grouped: next_out %d is null", i);
   }
   return gated_launch(groups, g, branch_dtype, width, eps, next ? next_out_dtype : IRIS_BF16, stream);

@@ -458,20 +458,21 @@ class HipIris:
         text = text.to(dev, torch.float32).contiguous()
         self._conditioning(ws, t.reshape(B).to(dev, torch.float32).contiguous())
         N = T + Lp
-        if cfg.block_kind(index) == "mmdit":
-            ws["X"].copy_(x.reshape(B * Lp, D))
-            ws["Y"].copy_(text.reshape(B * T, D))
-        else:
+        ws["block"] = (index, B, T, Lp, N)
+        if cfg.block_kind(index) != "mmdit" and not cfg.text_out(index):
             K.copy_rows(text.reshape(B * T, D), ws["tok"], B, T, 0, T, 0, N)
             K.copy_rows(x.reshape(B * Lp, D), ws["tok"], B, Lp, 0, Lp, T, N)
-        ws["block"] = (index, B, T, Lp, N)
-        self.run_block()
-        if cfg.block_kind(index) == "mmdit":
-            return ws["X"].view(B, Lp, D).clone(), ws["Y"].view(B, T, D).clone()
-        if not cfg.text_out(index):
+            self.run_block()
             return ws["X"].view(B, Lp, D).clone(), text
-        tok = ws["tok"].view(B, N, D)
-        return tok[:, T:].clone(), tok[:, :T].clone()
+        # the inputs enter the workspace's residual in the block's first kernels (the input norms) and
+        # leave it in its last
+        io = (x, text, torch.empty_like(x), torch.empty_like(text))
+        blk = self.blocks[index]
+        if blk["kind"] == "mmdit":
+            self._dual_block(ws, blk, B, T, Lp, N, False, None, io)
+        else:
+            self._single_block(ws, blk, B, T, Lp, N, False, False, None, io)
+        return io[2], io[3]
 
     def run_block(self) -> None:
         """Run the block of the last ``block_forward`` call again, in place on the residual it
@@ -490,10 +491,11 @@ class HipIris:
         return ws["mod_views"][table][index][chunk]
 
     def _dual_block(self, ws: dict, blk: dict, B: int, T: int, Lp: int, N: int, h_ready: bool,
-                    nxt: dict | None) -> None:
+                    nxt: dict | None, io: tuple | None = None) -> None:
         """One dual-stream block on the image ``X`` and text ``Y`` residuals. With ``h_ready`` the
         input norms are already in the ``h`` rows (fused into the previous block's last residual);
-        with ``nxt`` (a dual block) this block's last residual also produces ``nxt``'s input norms."""
+        with ``nxt`` (a dual block) this block's last residual also produces ``nxt``'s input norms.
+        With ``io`` (x, text, x_out, text_out) the streams come from and also go to the caller's tensors."""
         cfg, eps = self.cfg, self.eps
         D, H, Hkv = cfg.hidden_size, cfg.num_heads, cfg.kv_heads
         X, Y = ws["X"].view(B, Lp, D), ws["Y"].view(B, T, D)
@@ -507,7 +509,10 @@ class HipIris:
         hhx, hhy = ws["hh"][:rows_x], ws["hh"][rows_x:rows_x + rows_y]
         bf16 = torch.bfloat16
 
-        if not h_ready:
+        if io is not None:
+            K.rms_norm_modulate_copy(io[0], blk["norm_x1"], xm[0], xm[1], eps, hx, ws["X"], Lp)
+            K.rms_norm_modulate_copy(io[1], blk["norm_y1"], ym[0], ym[1], eps, hy, ws["Y"], T)
+        elif not h_ready:
             K.rms_norm_modulate(X, blk["norm_x1"], xm[0], xm[1], eps, bf16, out=hx.view(B, Lp, D))
             K.rms_norm_modulate(Y, blk["norm_y1"], ym[0], ym[1], eps, bf16, out=hy.view(B, T, D))
         # q | k | v | gate in one launch, the Q / K norm + rotary in the store of the q | k | v
@@ -527,7 +532,10 @@ class HipIris:
                                   [hx.view(B, Lp, D), hy.view(B, T, D)])
         K.linear_grouped([hx, hy], [blk["w13_x"], blk["w13_y"]], None, [hhx, hhy], swiglu=True)
         K.linear_grouped([hhx, hhy], [blk["w2_x"], blk["w2_y"]], None, [bx, by])
-        if nxt is None:
+        if io is not None:
+            K.gated_residual_copy_([X, Y], [bx.view(B, Lp, D), by.view(B, T, D)],
+                                   [blk["mlp_post_norm_x"], blk["mlp_post_norm_y"]], [xm[5], ym[5]], eps, io[2:])
+        elif nxt is None:
             K.gated_residual_grouped_([X, Y], [bx.view(B, Lp, D), by.view(B, T, D)],
                                       [blk["mlp_post_norm_x"], blk["mlp_post_norm_y"]], [xm[5], ym[5]], eps)
         else:
@@ -539,16 +547,20 @@ class HipIris:
                                       [hx.view(B, Lp, D), hy.view(B, T, D)])
 
     def _single_block(self, ws: dict, blk: dict, B: int, T: int, Lp: int, N: int, last: bool, h_ready: bool,
-                      nxt: dict | None) -> None:
+                      nxt: dict | None, io: tuple | None = None) -> None:
         """One single-stream block on ``tok`` (the last one continues on the image rows only).
-        ``h_ready`` / ``nxt``: as for ``_dual_block``, with ``nxt`` a single-stream block."""
+        ``h_ready`` / ``nxt`` / ``io``: as for ``_dual_block``, with ``nxt`` a single-stream block."""
         cfg, eps = self.cfg, self.eps
         D, H, Hkv = cfg.hidden_size, cfg.num_heads, cfg.kv_heads
         tok = ws["tok"]
         m = [self._mods(ws, "mods_img", blk["img_mod"], c) for c in range(6)]
         rows = B * N
         h, proj = ws["h_tok"][:rows], ws["qkvg"][:rows]
-        if not h_ready:
+        if io is not None:
+            if T:
+                K.rms_norm_modulate_copy(io[1], blk["norm1"], m[0], m[1], eps, h, tok, N)
+            K.rms_norm_modulate_copy(io[0], blk["norm1"], m[0], m[1], eps, h, tok, N, T)
+        elif not h_ready:
             K.rms_norm_modulate(tok.view(B, N, D), blk["norm1"], m[0], m[1], eps, torch.bfloat16, out=h.view(B, N, D))
         rope_c, rope_s = ws["rope"]
         q, k, vt = ws["q"], ws["k"], ws["vt"]
@@ -576,7 +588,10 @@ class HipIris:
                                         blk["norm2"], m[3], m[4], h2.view(B, per_batch, D))
         K.linear(h2, blk["w13"], out=hh, swiglu=True)
         K.linear(hh, blk["w2"], out=branch)
-        if nxt is None:
+        if io is not None:
+            K.gated_residual_copy_([Rv], [branch.view(B, per_batch, D)], [blk["mlp_post_norm"]], [m[5]], eps,
+                                   [(io[3], io[2])])
+        elif nxt is None:
             K.gated_residual_rms_norm_(Rv, branch.view(B, per_batch, D), blk["mlp_post_norm"], m[5], eps)
         else:
             n1 = [self._mods(ws, "mods_img", nxt["img_mod"], c) for c in range(2)]

@@ -241,6 +241,53 @@ def gated_residual_grouped_(residuals, branches, weights, gates, eps: float, nex
     )
 
 
+def rms_norm_modulate_copy(x, weight, shift, scale, eps: float, out, copy, dst_batch_rows: int, dst_offset: int = 0):
+    """``rms_norm_modulate`` of FP32 ``x`` ``[B, N, D]`` into rows ``b * dst_batch_rows + dst_offset + n`` of
+    ``out`` (``[rows, D]``), and ``x`` itself into those rows of the FP32 ``copy``, in one pass."""
+    batch, tokens, width = x.shape
+    check = _Check("rms_norm_modulate_copy", x, weight, shift, scale, out, copy)
+    check(width % 128 == 0, f"needs a width that is a multiple of 128 (got {width})")
+    check.fp32(x=x, copy=copy).gains(width, weight=weight)
+    check(out.is_contiguous() and out.shape[-1] == copy.shape[-1] == width
+          and min(out.numel(), copy.numel()) >= batch * dst_batch_rows * width
+          and 0 <= dst_offset <= dst_batch_rows - tokens, "out or copy does not cover the rows")
+    shift, scale, stride = _mod_pair(shift, scale, batch, width)
+    L.call("iris_rms_norm_modulate_copy", L.ptr(x), L.ptr(out), L.dtype_code(out.dtype), L.ptr(copy), L.ptr(weight),
+           L.ptr(shift), L.ptr(scale), batch * tokens, tokens, width, stride, float(eps), dst_batch_rows, dst_offset,
+           L.stream())
+
+
+def gated_residual_copy_(residuals, branches, weights, gates, eps: float, copies) -> None:
+    """``gated_residual_rms_norm_`` of one or two streams ``[B, N, D]`` whose updated rows are also written
+    to ``copies[i]``: one packed FP32 tensor of the stream's shape, or a pair of them, ``[B, S, D]`` and
+    ``[B, N - S, D]``, holding the first ``S`` tokens of each item and the rest."""
+    width = residuals[0].shape[-1]
+    gate_rows, first, rest, splits = [], [], [], []
+    for residual, branch, weight, gate, copy in zip(residuals, branches, weights, gates, copies):
+        batch, tokens, w = residual.shape
+        pair = copy if isinstance(copy, tuple) else (None, copy)
+        check = _Check("gated_residual_copy_", residual, branch, weight, gate, *pair)
+        check(w == width and branch.dtype == branches[0].dtype, "the streams differ in width or branch dtype")
+        _residual_checks(check, residual, branch, width)
+        check.gains(width, weight=weight)
+        split = 0 if pair[0] is None else pair[0].shape[1]
+        check(split < tokens and pair[1].shape == (batch, tokens - split, width)
+              and (pair[0] is None or pair[0].shape == (batch, split, width)), "copies do not match the stream")
+        check.fp32(**{f"copy{i}": c for i, c in enumerate(pair) if c is not None})
+        gate_rows.append(_mod_rows(gate, batch, width))
+        first.append(pair[0])
+        rest.append(pair[1])
+        splits.append(split)
+    P = L.pointer_array
+    L.call(
+        "iris_gated_residual_copy", len(residuals), P([L.ptr(r) for r in residuals]), P([L.ptr(b) for b in branches]),
+        L.dtype_code(branches[0].dtype), P([L.ptr(w) for w in weights]), P([L.ptr(g) for g, _ in gate_rows]),
+        L.long_array([r.shape[0] * r.shape[1] for r in residuals]), L.long_array([r.shape[1] for r in residuals]), width,
+        L.long_array([stride for _, stride in gate_rows]), float(eps), P([L.ptr(c) for c in first]),
+        P([L.ptr(c) for c in rest]), L.long_array(splits), L.stream(),
+    )
+
+
 def pixel_rms_norm(pixels: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """``rms_norm(pixels) * weight`` over the 16 channels of each pixel, stored BF16
     (src/iris_metal/kernels.py:486-498)."""

@@ -104,3 +104,33 @@ def test_residual_rms_norm_rows(width, rows):
             if extra is not None:
                 want = want + extra.double()[torch.arange(rows, device=DEV) % 3]
             torch.testing.assert_close(out.double(), want, rtol=2e-6, atol=4e-6)
+
+
+@pytest.mark.parametrize("width", [128, 2560])
+@pytest.mark.parametrize("batch,text,image", [(1, 3, 70), (2, 77, 240), (2, 1, 1000)])
+def test_rows_enter_and_leave_a_residual_stream(width, batch, text, image):
+    """``rms_norm_modulate_copy`` of text and image rows into one joined stream is the copies followed by
+    ``rms_norm_modulate``; ``gated_residual_copy_`` is the residual followed by the copies (2 x 1001 rows:
+    the wave form)."""
+    g = torch.Generator(device=DEV).manual_seed(74)
+    n = text + image
+    rows = torch.randn(batch, n, width, generator=g, device=DEV)
+    w = 1 + 0.1 * torch.randn(width, generator=g, device=DEV)
+    shift, scale, gate = (0.1 * torch.randn(batch, 1, width, generator=g, device=DEV) for _ in range(3))
+    stream = torch.full((batch * n, width), 5.0, device=DEV)
+    h = torch.empty(batch * n, width, device=DEV, dtype=torch.bfloat16)
+    K.rms_norm_modulate_copy(rows[:, :text].contiguous(), w, shift, scale, 1e-6, h, stream, n)
+    K.rms_norm_modulate_copy(rows[:, text:].contiguous(), w, shift, scale, 1e-6, h, stream, n, text)
+    assert torch.equal(stream.view(batch, n, width), rows)
+    assert torch.equal(h.view(batch, n, width), K.rms_norm_modulate(rows, w, shift, scale, 1e-6, torch.bfloat16))
+    want = K.gated_residual_rms_norm_(rows.clone(), h.view_as(rows), w, gate, 1e-6)
+    first, rest = (torch.empty(batch, m, width, device=DEV) for m in (text, image))
+    got, whole = stream.view(batch, n, width), torch.empty_like(rows)
+    again = got.clone()
+    K.gated_residual_copy_([got], [h.view_as(rows)], [w], [gate], 1e-6, [(first, rest)])
+    assert torch.equal(got, want) and torch.equal(torch.cat([first, rest], 1), want)
+    other = [again, rows[:, :text].contiguous()]
+    K.gated_residual_copy_(other, [h.view_as(rows), h.view_as(rows)[:, :text].contiguous()], [w, w], [gate, gate], 1e-6,
+                           (whole, first))
+    assert torch.equal(again, want) and torch.equal(whole, want)
+    assert torch.equal(other[1], want[:, :text]) and torch.equal(first, want[:, :text])
