@@ -1761,6 +1761,10 @@ struct RingTile {
 };
 constexpr RingTile kRingTiles[] = {{18, 0.158, 5.5}, {19, 0.166, 6.4}, {20, 0.219, 6.3}, {21, 0.275, 8.8}, {22, 0.225, 9.2},
                                    {23, 0.290, 9.5}, {24, 0.345, 10.0}, {25, 0.450, 9.5}, {26, 0.545, 9.5}};
+// Ring launches of several rounds run further above the model inside a forward than the four-wave ones
+// (SwiGLU of 256 + 77 rows, 428 tiles of 96 x 128 in two rounds: 44 us alone, 56 in the forward, where
+// 162 tiles of 192 x 256 in one take 49), so they must win by as much.
+constexpr double kRingRounds = 1.1;
 // The four-wave tiles in the same terms: tile area / (rate x this) per K tile, a first round's and a
 // further round's extra (the next tile's loads overlap a persistent round's output), and what the
 // q|k|v store adds to its launch.
@@ -1809,7 +1813,7 @@ int pick_ring(const int* m, int groups, int n, int k, int epilogue, double& us) 
   for (const RingTile& r : kRingTiles) {
     if (!ring_allowed(r.tile, k, epilogue)) continue;
     const long rounds = (launch_tiles(kTiles[r.tile], m, groups, n) + cus - 1) / cus;
-    const double cost = rounds * (k / kBK * r.ktile_us + r.fixed_us);
+    const double cost = rounds * (k / kBK * r.ktile_us + r.fixed_us) * (rounds > 1 ? kRingRounds : 1.0);
     if (cost < us) best = r.tile, us = cost;
   }
   return best;
