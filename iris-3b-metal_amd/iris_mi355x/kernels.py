@@ -735,6 +735,7 @@ def gemv(
 def gemv_pair(weights, x: torch.Tensor, biases, outs, extra_biases, in_silu: bool = False) -> None:
     """``gemv`` with extra biases of two weights on the same inputs (the image and text adaLN cores)
     in one launch; same results as the two calls."""
+    _Check("gemv_pair")(len(weights) == len(biases) == len(outs) == len(extra_biases) == 2, "takes two products")
     batch, k = x.shape
     for w, b, o, e in zip(weights, biases, outs, extra_biases):
         check = _Check("gemv_pair", w, x, b, o, e)

@@ -24,6 +24,14 @@ def test_cpu_tensors_are_refused():
         K.pixel_rms_norm(torch.zeros(1, 1, 16), torch.ones(16), 1e-6)
 
 
+@pytest.mark.parametrize("lengths", [(0, 0, 0, 0), (1, 1, 1, 1), (2, 1, 2, 2), (2, 2, 1, 2), (2, 2, 2, 1), (3, 3, 3, 3)])
+def test_gemv_pair_takes_two_products(lengths):
+    """Checked before the device and the tensors: the library reads two entries of every list."""
+    weights, biases, outs, extras = ([torch.zeros(1)] * n for n in lengths)
+    with pytest.raises(ValueError, match="gemv_pair: takes two products"):
+        K.gemv_pair(weights, torch.zeros(1, 8), biases, outs, extras)
+
+
 @pytest.mark.gpu
 def test_kernels_reject_non_fp32_gains():
     x = torch.randn(1, 4, 128, device="cuda")
