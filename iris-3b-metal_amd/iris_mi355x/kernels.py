@@ -261,6 +261,10 @@ def gated_residual_copy_(residuals, branches, weights, gates, eps: float, copies
     """``gated_residual_rms_norm_`` of one or two streams ``[B, N, D]`` whose updated rows are also written
     to ``copies[i]``: one packed FP32 tensor of the stream's shape, or a pair of them, ``[B, S, D]`` and
     ``[B, N - S, D]``, holding the first ``S`` tokens of each item and the rest."""
+    groups = len(residuals)
+    _Check("gated_residual_copy_")(
+        groups in (1, 2) and len(branches) == len(weights) == len(gates) == len(copies) == groups
+        and all(len(c) == 2 for c in copies if isinstance(c, tuple)), "takes one or two streams")
     width = residuals[0].shape[-1]
     gate_rows, first, rest, splits = [], [], [], []
     for residual, branch, weight, gate, copy in zip(residuals, branches, weights, gates, copies):
@@ -280,7 +284,7 @@ def gated_residual_copy_(residuals, branches, weights, gates, eps: float, copies
         splits.append(split)
     P = L.pointer_array
     L.call(
-        "iris_gated_residual_copy", len(residuals), P([L.ptr(r) for r in residuals]), P([L.ptr(b) for b in branches]),
+        "iris_gated_residual_copy", groups, P([L.ptr(r) for r in residuals]), P([L.ptr(b) for b in branches]),
         L.dtype_code(branches[0].dtype), P([L.ptr(w) for w in weights]), P([L.ptr(g) for g, _ in gate_rows]),
         L.long_array([r.shape[0] * r.shape[1] for r in residuals]), L.long_array([r.shape[1] for r in residuals]), width,
         L.long_array([stride for _, stride in gate_rows]), float(eps), P([L.ptr(c) for c in first]),

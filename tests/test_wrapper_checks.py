@@ -32,6 +32,15 @@ def test_gemv_pair_takes_two_products(lengths):
         K.gemv_pair(weights, torch.zeros(1, 8), biases, outs, extras)
 
 
+@pytest.mark.parametrize("lengths", [(0, 0, 0, 0, 0), (2, 1, 2, 2, 2), (2, 2, 1, 2, 2), (2, 2, 2, 1, 2), (2, 2, 2, 2, 1),
+                                     (1, 2, 2, 2, 2), (3, 3, 3, 3, 3)])
+def test_gated_residual_copy_takes_one_or_two_whole_streams(lengths):
+    """Checked before the device and the tensors: the library reads one entry of every list per stream."""
+    residuals, branches, weights, gates, copies = ([torch.zeros(1, 1, 128)] * n for n in lengths)
+    with pytest.raises(ValueError, match="gated_residual_copy_: takes one or two streams"):
+        K.gated_residual_copy_(residuals, branches, weights, gates, 1e-6, copies)
+
+
 @pytest.mark.gpu
 def test_kernels_reject_non_fp32_gains():
     x = torch.randn(1, 4, 128, device="cuda")
