@@ -460,7 +460,8 @@ def linear(
 
 def linear_grouped(xs, weights, biases, outs, swiglu: bool = False) -> None:
     """Two ``linear`` calls of equal weight shape (one per stream of a dual block) in one launch."""
-    _Check("linear_grouped")(len(xs) == len(weights) == len(outs) == 2, "takes two problems")
+    _Check("linear_grouped")(len(xs) == len(weights) == len(outs) == 2 and (biases is None or len(biases) == 2),
+                             "takes two problems")
     k = xs[0].shape[-1]
     n = weights[0].shape[0]
     for x, w, o in zip(xs, weights, outs):

@@ -41,6 +41,13 @@ def test_gated_residual_copy_takes_one_or_two_whole_streams(lengths):
         K.gated_residual_copy_(residuals, branches, weights, gates, 1e-6, copies)
 
 
+@pytest.mark.parametrize("lengths", [(2, 2, 0, 2), (2, 2, 1, 2), (2, 2, 3, 2), (1, 2, 2, 2)])
+def test_linear_grouped_takes_two_problems(lengths):
+    xs, weights, biases, outs = ([torch.zeros(1, 64)] * n for n in lengths)
+    with pytest.raises(ValueError, match="linear_grouped: takes two problems"):
+        K.linear_grouped(xs, weights, biases, outs)
+
+
 @pytest.mark.gpu
 def test_kernels_reject_non_fp32_gains():
     x = torch.randn(1, 4, 128, device="cuda")
