@@ -2123,7 +2123,8 @@ static int qk_rope_gemm(bool any_rows, int groups, const void* const* a, const v
   // the 256 x 256 store transposes whole 256-row items only: otherwise the V columns go to c and from
   // there to vt in a launch of their own
   bool whole = true;
-  for (int i = 0; i < groups; ++i) whole = whole && rows_per_batch[i] % 256 == 0 && dst_offset[i] % 16 == 0;
+  for (int i = 0; i < groups; ++i)
+    whole = whole && (m[i] == 0 || (rows_per_batch[i] % 256 == 0 && dst_offset[i] % 16 == 0));
   if (vt && !whole) {
     const int rc = qk_rope_gemm(false, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch,
                                 dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, nullptr,

@@ -135,6 +135,29 @@ def test_qkv_of_any_rows_without_ring_tiles(tokens, batch):
         assert torch.equal(got, want)
 
 
+def test_qk_store_of_whole_items_beside_an_empty_ragged_group():
+    """Without rows a group's batch items do not matter: the 256 x 256 store still writes V^T itself and
+    leaves the V columns of the output alone."""
+    g = torch.Generator(device=DEV).manual_seed(48)
+    k, n = 256, 6 * 128
+    x, w = randn(g, 256, k), randn(g, n, k, scale=0.05)
+    gain, cos, sin = torch.ones(128, device=DEV), *(torch.randn(256, 64, generator=g, device=DEV) for _ in range(2))
+    plain = forced(16, lambda: K.linear(x, w))
+    bufs = [[torch.full((1, h, *s), 3.0, device=DEV, dtype=torch.bfloat16)
+             for h, s in ((2, (256, 128)), (1, (256, 128)), (1, (128, 256)))] for _ in range(2)]
+    K.qkv_prepare(plain.view(1, 256, n), gain, gain, cos, sin, 1e-6, 2, 1, *bufs[0], 0, 256, 384)
+    out = torch.full((256, n), 5.0, device=DEV, dtype=torch.bfloat16)
+    P, q, key, vt = _lib.pointer_array, *bufs[1]
+    twice = [P([t.data_ptr()] * 2) for t in (x, w, out, gain)]
+    forced(16, lambda: _lib.call(
+        "iris_gemm_bf16_qk_rope", 2, *twice[:3], _lib.int_array([256, 0]), n, k, k, k, n, twice[3], twice[3],
+        _lib.int_array([256, 77]), _lib.int_array([0, 0]), cos.data_ptr(), sin.data_ptr(), 256, q.data_ptr(),
+        key.data_ptr(), 2, 1, 256, vt.data_ptr(), 256, 1e-6, _lib.stream()))
+    for got, want in zip(bufs[1], bufs[0]):
+        assert torch.equal(got, want)
+    assert torch.all(out[:, :512] == 5.0) and torch.equal(out[:, 512:], plain[:, 512:])
+
+
 def test_ring_refuses_a_k_loop_shorter_than_its_ring():
     x, w = torch.zeros(8, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(64, 128, device=DEV, dtype=torch.bfloat16)
     with pytest.raises(Exception, match="ring"):
