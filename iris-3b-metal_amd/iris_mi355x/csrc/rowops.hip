@@ -69,7 +69,15 @@ __device__ __forceinline__ float split_row_sum(float chunk, float (&part)[NC][kW
 // width 2560 with every buffer from HBM, split / wave per row: gated residual with the next norm 333
 // rows 6.8 / 7.7, 1280: 13.4 / 15.8, 1848: 18.9 / 18.8; modulate FP32 333: 4.3 / 5.0, 1280: 7.3 / 7.8,
 // 1848: 10.0 / 9.4; modulate BF16 333: 4.0 / 4.6, 640: 4.9 / 4.6, 4352: 16.2 / 12.3.
-constexpr long kGatedSplitRows = 1792;
+// The gated residual's wave form gains more where the next norm's coefficients are read once per four
+// rows (`shared`), and with three chunks per lane also without: there it takes over at 1408 rows, us
+// split / wave with the next norm, BF16 branch: 2560 wide, shared, 1408 rows 15.6 / 15.7, 1792: 18.6 /
+// 17.2 (1791, not shared: 18.4 / 19.1); 4096 wide 1408: 19.9 / 20.6, 1792: 24.2 / 22.6; 1536 wide 1280:
+// 8.1 / 9.0, 1663, not shared: 11.5 / 10.7. Up to two chunks the split form stays ahead (1024 wide, 1792
+// rows: 7.2 / 7.5).
+long gated_split_rows(int nc, bool next, bool shared) {
+  return next && (nc == 3 || (nc > 3 && shared)) ? 1408 : 1792;
+}
 long modulate_split_rows(int x_dtype) { return x_dtype == IRIS_F32 ? 1536 : 512; }
 
 // NC = 8-element chunks each lane holds (width <= NC * 512). A wave issues its row's loads
@@ -680,12 +688,13 @@ int gated_launch(int groups, const GatedGroup* g, int branch_dtype, int width, f
   a.eps = eps;
   if (rows == 0) return IRIS_OK;
   IRIS_REQUIRE(rows < (1L << 31), "gated_residual_rms_norm: too many rows");
-  if (rows > kGatedSplitRows) {
+  // with the next norm, coefficients in LDS when every workgroup's four rows share a batch
+  // index (without it the LDS fill and its barrier cost more than the one coefficient row saves)
+  const bool next = g[0].next_out != nullptr;
+  bool shared = next && 3L * width * sizeof(float) <= 48 * 1024;
+  for (int i = 0; i < groups; ++i) shared = shared && g[i].rows_per_batch % kRowsPerBlock == 0;
+  if (rows > gated_split_rows(nc_bucket(width), next, shared)) {
     const dim3 grid(static_cast<unsigned>((a.rows0 + 3) / 4 + (groups > 1 ? (g[1].rows + 3) / 4 : 0)));
-    // with the next norm, coefficients in LDS when every workgroup's four rows share a batch
-    // index (without it the LDS fill and its barrier cost more than the one coefficient row saves)
-    bool shared = g[0].next_out != nullptr && 3L * width * sizeof(float) <= 48 * 1024;
-    for (int i = 0; i < groups; ++i) shared = shared && g[i].rows_per_batch % kRowsPerBlock == 0;
     IRIS_NC_DISPATCH(nc_bucket(width), {
       if (branch_dtype == IRIS_BF16)
         launch_gated<NC, bf16>(grid, stream, a, out_dtype, shared);

@@ -87,6 +87,33 @@ def test_gated_residual_forms_agree(width, rows):
         assert torch.equal(part, got[:, :n]) and torch.equal(part_out, out[:, :n])
 
 
+@pytest.mark.parametrize("width", [*WIDTHS, 1408])
+@pytest.mark.parametrize("rows,part", [((1412,), 1408), ((1411,), 1408), ((1200, 212), 1408)])
+def test_gated_residual_forms_agree_around_the_shared_limit(width, rows, part):
+    """With the next norm the wave form takes over earlier where four rows share its coefficients (1412
+    rows, also of two streams) or a lane holds three chunks (1025 to 1536 columns): the same bits as the
+    first 1408 rows in one launch."""
+    g = torch.Generator(device=DEV).manual_seed(75)
+    n = sum(rows)
+    res, br = (torch.randn(1, n, width, generator=g, device=DEV) for _ in range(2))
+    w, w2 = (1 + 0.1 * torch.randn(width, generator=g, device=DEV) for _ in range(2))
+    gate, shift, scale = (0.1 * torch.randn(1, 1, width, generator=g, device=DEV) for _ in range(3))
+
+    def run(*parts):
+        r = [t.clone() for t in (res[:, a:b] for a, b in parts)]
+        b = [br[:, a:b].contiguous() for a, b in parts]
+        o = [torch.empty_like(t) for t in r]
+        if len(parts) == 1:
+            K.gated_residual_norm_modulate_(r[0], b[0], w, gate, 1e-6, w2, shift, scale, o[0])
+        else:
+            K.gated_residual_grouped_(r, b, [w] * 2, [gate] * 2, 1e-6, [w2] * 2, [shift] * 2, [scale] * 2, o)
+        return torch.cat(r, 1), torch.cat(o, 1)
+
+    whole = run((0, n)) if len(rows) == 1 else run((0, rows[0]), (rows[0], n))
+    for got, want in zip(whole, run((0, part))):
+        assert torch.equal(got[:, :part], want)
+
+
 @pytest.mark.parametrize("width", [8, 264, *WIDTHS])
 @pytest.mark.parametrize("rows", [1, 7, 130])
 def test_residual_rms_norm_rows(width, rows):
