@@ -1806,12 +1806,13 @@ double pair_us(int tile1, int n1, double extra1, int tile2, int n2, const int* m
   return (work + 0.5 * t2 > longest ? work + 0.5 * t2 : longest) + kFirstRoundUs;
 }
 
-// The ring tile that runs the launch in less than `us` (which it then lowers to its time), or -1.
-int pick_ring(const int* m, int groups, int n, int k, int epilogue, double& us) {
+// The ring tile of at most `max_area` that runs the launch in less than `us` (which it then lowers to its
+// time), or -1.
+int pick_ring(const int* m, int groups, int n, int k, int epilogue, double& us, int max_area = 1 << 30) {
   int best = -1;
   const int cus = device_cus();
   for (const RingTile& r : kRingTiles) {
-    if (!ring_allowed(r.tile, k, epilogue)) continue;
+    if (!ring_allowed(r.tile, k, epilogue) || kTiles[r.tile].bm * kTiles[r.tile].bn > max_area) continue;
     const long rounds = (launch_tiles(kTiles[r.tile], m, groups, n) + cus - 1) / cus;
     const double cost = rounds * (k / kBK * r.ktile_us + r.fixed_us) * (rounds > 1 ? kRingRounds : 1.0);
     if (cost < us) best = r.tile, us = cost;
@@ -1828,7 +1829,12 @@ SplitPlan plan_mfma16(const int* m, int groups, int n, int k, int epilogue) {
   double us = plan.n1 == 0 ? four_wave_us(plan.tile1, m, groups, n, k)
                            : four_wave_us(plan.tile1, m, groups, plan.n1, k) +
                                  four_wave_us(plan.tile2, m, groups, n - plan.n1, k) - kFirstRoundUs + kNextRoundUs;
-  const int ring = pick_ring(m, groups, n, k, epilogue, us);
+  // A ring tile larger than the four-wave tile of a one-round plan has more work per CU, whatever the
+  // model says of short K loops: 192 x 128 against 128 x 160, us at 1280 x 3840, K = 512 11.3 / 10.5, 1024:
+  // 16.4 / 14.6, 1280: 20.6 / 18.6, 4096: 49 / 47; 4096 x 1280 x 1280 20.6 / 18.9.
+  const TileShape four_wave = kTiles[plan.tile1];
+  const bool one_round = plan.n1 == 0 && launch_tiles(four_wave, m, groups, n) <= device_cus();
+  const int ring = pick_ring(m, groups, n, k, epilogue, us, one_round ? four_wave.bm * four_wave.bn : 1 << 30);
   if (ring >= 0) plan = SplitPlan{0, ring, ring};
   const int square = kCandidates[kSquare].tile;
   const long row_tiles = launch_tiles(kTiles[square], m, groups, kTiles[square].bn);
