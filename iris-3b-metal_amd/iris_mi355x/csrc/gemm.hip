@@ -1783,6 +1783,11 @@ long launch_tiles(const TileShape& t, const int* m, int groups, int n) {
   return tiles;
 }
 
+// Output area of a launch's tiles, padding included.
+double tile_area(int tile, const int* m, int groups, int n) {
+  return static_cast<double>(launch_tiles(kTiles[tile], m, groups, n)) * kTiles[tile].bm * kTiles[tile].bn;
+}
+
 // K loop of one four-wave tile.
 double four_wave_tile_us(int tile, int k) {
   double rate = 1.0;
@@ -1836,17 +1841,31 @@ SplitPlan plan_mfma16(const int* m, int groups, int n, int k, int epilogue) {
   const bool one_round = plan.n1 == 0 && launch_tiles(four_wave, m, groups, n) <= device_cus();
   const int ring = pick_ring(m, groups, n, k, epilogue, us, one_round ? four_wave.bm * four_wave.bn : 1 << 30);
   if (ring >= 0) plan = SplitPlan{0, ring, ring};
+  // SwiGLU's columns left over: a tail of 192 x 128 tiles measured level to 4% slower than the four-wave
+  // plans (3600 x 5504 x 1280: 55 us against 53); and in a long call, held by the power limit, padded rows
+  // cost time in every round, so there the estimate grows with the tiles' area over the plan's to beat and
+  // must win by 1% (13696 columns, K = 2560, us tail / four-wave: 3586 rows 225 / 222, 4992: 295 / 289, 5890:
+  // 349 / 343; the plans kept: 5000 rows 292 / 301, 6144: 349 / 357, 8704: 488 / 499). Plain tails were
+  // 3 to 15% ahead wherever the model takes them (6402 x 2560 x 6848: 197 / 226).
+  const bool swiglu = epilogue == IRIS_EPI_SILU_MUL;
   const int square = kCandidates[kSquare].tile;
   const long row_tiles = launch_tiles(kTiles[square], m, groups, kTiles[square].bn);
+  double area = plan.n1 == 0 ? tile_area(plan.tile1, m, groups, n)
+                             : tile_area(plan.tile1, m, groups, plan.n1) + tile_area(plan.tile2, m, groups, n - plan.n1);
   for (long rounds = 1; row_tiles > 0; ++rounds) {
-    const long n1 = rounds * device_cus() / row_tiles * 256;
-    if (n1 >= n) break;
-    if (n1 == 0) continue;
-    const double first = four_wave_us(square, m, groups, static_cast<int>(n1), k);
+    const long whole = rounds * device_cus() / row_tiles * 256;
+    if (whole >= n) break;
+    if (whole == 0) continue;
+    const int n1 = static_cast<int>(whole);
+    const double first = four_wave_us(square, m, groups, n1, k);
     if (first >= us) break;
     double rest = us - first;
-    const int tail = pick_ring(m, groups, n - static_cast<int>(n1), k, epilogue, rest);
-    if (tail >= 0) plan = SplitPlan{static_cast<int>(n1), square, tail}, us = first + rest;
+    const int tail = pick_ring(m, groups, n - n1, k, epilogue, rest, swiglu ? 128 * 128 : 1 << 30);
+    if (tail < 0) continue;
+    const double tail_area = tile_area(square, m, groups, n1) + tile_area(tail, m, groups, n - n1);
+    const double padding = tail_area > area ? tail_area / area : 1.0;
+    if (swiglu && k >= 2048 && rounds >= 3 && (first + rest) * padding >= 0.99 * us) continue;
+    plan = SplitPlan{n1, square, tail}, us = first + rest, area = tail_area;
   }
   return plan;
 }

@@ -173,3 +173,13 @@ def test_automatic_choice_over_row_counts_is_row_independent(n, k, swiglu):
     whole = K.linear(x, w, swiglu=swiglu)
     for m in (1, 40, 130, 333, 520, 900):
         assert torch.equal(K.linear(x[:m], w, swiglu=swiglu), whole[:m])
+
+
+@pytest.mark.parametrize("m,n,k,swiglu", [(1280, 3840, 512, False), (1153, 4096, 1280, False), (4097, 4096, 1280, False),
+                                          (3586, 13696, 2560, True), (5000, 13696, 2560, True), (3590, 5504, 1280, True)])
+def test_automatic_plans_are_the_four_wave_tile_bit_for_bit(m, n, k, swiglu):
+    """On either side of the plan rules: one round of ring or four-wave tiles, columns left over after whole
+    rounds on ring tiles or in a pair."""
+    g = torch.Generator(device=DEV).manual_seed(49)
+    x, w = randn(g, m, k), randn(g, n, k, scale=0.02)
+    assert torch.equal(K.linear(x, w, swiglu=swiglu), forced(16, lambda: K.linear(x, w, swiglu=swiglu)))
