@@ -1769,6 +1769,7 @@ constexpr double kRingRounds = 1.1;
 // further round's extra (the next tile's loads overlap a persistent round's output), and what the
 // q|k|v store adds to its launch.
 constexpr double kAreaPerUs = 48600.0, kFirstRoundUs = 11.0, kNextRoundUs = 5.0, kQkStoreUs = 9.0;
+constexpr double kPairTurnUs = 8.0;  // a pair's tiles are workgroups of their own, without that overlap
 
 bool ring_allowed(int tile, int k, int epilogue) {
   const TileShape t = kTiles[tile];
@@ -1809,6 +1810,28 @@ double pair_us(int tile1, int n1, double extra1, int tile2, int n2, const int* m
   const double work = (launch_tiles(kTiles[tile1], m, groups, n1) * t1 + launch_tiles(kTiles[tile2], m, groups, n2) * t2) /
                       device_cus();
   return (work + 0.5 * t2 > longest ? work + 0.5 * t2 : longest) + kFirstRoundUs;
+}
+
+// When the last tile of two GEMMs in one launch ends, where the first's tiles fit one round: each tile with
+// its own first K tiles and output, the second's on whichever CU is free next. pair_us is too hopeful where
+// the second needs a turn after the first's: 8 query and 8 K/V heads with gates, K = 1024: 4096 rows (192 +
+// 105 tiles, the second's in two turns on the CUs that the first leaves free) 49 us against 60 in two
+// launches, 4352 rows (204 + 112, a third turn) 63 against 59. (With more rounds of the first the launch is
+// held by the work: 20 and 5 heads, K = 2560, 4396 rows level, 5000 rows 171 against 205.)
+double pair_end_us(int tile1, int n1, double extra1, int tile2, int n2, const int* m, int groups, int k) {
+  const long cus = device_cus(), busy = launch_tiles(kTiles[tile1], m, groups, n1);
+  if (busy > cus) return 0.0;
+  const double turn = four_wave_tile_us(tile2, k) + kPairTurnUs;
+  double end_free = 0.0, end_busy = four_wave_tile_us(tile1, k) + extra1 + kFirstRoundUs;
+  double end = end_busy;
+  for (long left = launch_tiles(kTiles[tile2], m, groups, n2); left > 0;) {
+    const bool on_free = busy == 0 || (busy < cus && end_free <= end_busy);
+    double& next = on_free ? end_free : end_busy;
+    next += turn;
+    left -= on_free ? cus - busy : busy;
+    end = next > end ? next : end;
+  }
+  return end;
 }
 
 // The ring tile of at most `max_area` that runs the launch in less than `us` (which it then lowers to its
@@ -2136,7 +2159,8 @@ static int qk_rope_gemm(bool any_rows, int groups, const void* const* a, const v
       tile2 = pick_tile(m, groups, n - n_qkv, IRIS_EPI_NONE, -1);
       us += four_wave_us(tile2, m, groups, n - n_qkv, k);
       const double paired = pair_us(kQkRopeTile, n_qkv, kQkStoreUs, kQkPairTile, n - n_qkv, m, groups, k);
-      if (paired < us) tile2 = kQkPairTile, us = paired;
+      if (paired < us && pair_end_us(kQkRopeTile, n_qkv, kQkStoreUs, kQkPairTile, n - n_qkv, m, groups, k) < us)
+        tile2 = kQkPairTile, us = paired;
     }
     ring = pick_ring(m, groups, n, k, kEpiQkRope, us);
   } else {
