@@ -319,6 +319,36 @@ def test_iris3b_block_at_1024_matches_oracle(iris3b_full, iris3b_full_weights, i
         check(got.cpu() - before, want - before, f"block {index} {name} update")
 
 
+@pytest.mark.parametrize("index", [0, 8])
+@pytest.mark.parametrize("grid,n_text", [((13, 21), 77), ((29, 41), 131)])
+def test_iris3b_block_of_two_ragged_items_matches_oracle(iris3b_full, iris3b_full_weights, index, grid, n_text):
+    """A dual- and a single-stream block on two images of 273 or 1189 patches with 77 or 131 text
+    tokens (2640 joint rows of two items: the q | k | v store paired with the gate columns), against
+    the oracle block and bit for bit against each item alone."""
+    _, sd = iris3b_full_weights
+    cfg = IRIS_3B
+    g = torch.Generator().manual_seed(14)
+    s = torch.randn(2, grid[0] * grid[1], cfg.hidden_size, generator=g)
+    text = torch.randn(2, n_text, cfg.hidden_size, generator=g)
+    t = torch.tensor([700.0, 250.0])
+    got_x, got_y = iris3b_full.block_forward(index, s.to(DEV), text.to(DEV), t.to(DEV), grid)
+    for i in range(2):
+        one = slice(i, i + 1)
+        alone = iris3b_full.block_forward(index, s[one].to(DEV), text[one].to(DEV), t[one].to(DEV), grid)
+        assert torch.equal(alone[0], got_x[one]) and torch.equal(alone[1], got_y[one])
+    _all_cores()
+    cond = torch.nn.functional.silu(O.timestep_embed(sd, t, cfg.timestep_max_period))
+    img, txt, _ = O.rope_tables(cfg, grid, n_text)
+    if cfg.block_kind(index) == "mmdit":
+        want_x, want_y = O.mmdit_block(sd, cfg, index, s, text, cond, img, txt)
+    else:
+        tokens = O.single_block(sd, cfg, index, torch.cat([text, s], dim=1), n_text, cond, img, txt)
+        want_x, want_y = tokens[:, n_text:], tokens[:, :n_text]
+    for name, got, want, before in (("x", got_x, want_x, s), ("text", got_y, want_y, text)):
+        check(got, want, f"block {index} {name}")
+        check(got.cpu() - before, want - before, f"block {index} {name} update")
+
+
 def test_iris3b_full_size_batch_of_four_is_four_single_forwards(iris3b_full):
     """The guided workload's shape at full size (1024x1024, 4352 joint tokens, PiT over 1M pixels
     per image, batch 4 = two prompts with conditional and zero unconditional text), checked by a

@@ -601,11 +601,11 @@ def test_flash_attention_32_key_variants_agree_bitwise(n):
         assert torch.equal(outs[0], outs[i]), f"variant {(1, 3, 4)[i]} differs from variant 1"
 
 
-@pytest.mark.parametrize("n", [1000, 4352])
+@pytest.mark.parametrize("n", [1000, 2009, 4352])
 def test_flash_attention_batch_rows_do_not_depend_on_the_batch(n):
-    """20 query / 5 K/V heads: a batch of four gives each item the bits it gets alone (the
-    automatic variant follows one item's shape: at 1000 tokens a batch-sized grid would have
-    chosen the 16 x 16 x 32 form, which rounds differently from the single item's)."""
+    """20 query / 5 K/V heads: a batch of four gives each item the bits it gets alone. The automatic
+    variant follows one item's shape (on 256 CUs variant 2 at 1000 tokens, 6 at 2009, 5 at 4352),
+    where a rule on the whole grid would take another one for four items, which rounds differently."""
     b, h, hkv = 4, 20, 5
     q, k, v, qd, kd, vt = _attn_inputs(b, h, hkv, n, 23)
     out = torch.zeros(b * n, h * 128, device=DEV, dtype=torch.bfloat16)
@@ -673,6 +673,39 @@ def test_flash_attention_trunk_shape_with_gate_and_split(variant):
         gates = torch.sigmoid(gate[sel, hh * 128:(hh + 1) * 128].float())
         close_attention(got[sel, hh], plain * gates)
         close_attention(got[sel, hh] / gates, plain)  # the gate does not hide an error
+
+
+@pytest.mark.parametrize("b,t,l,variant", [(1, 77, 256, 2), (2, 77, 256, 2), (1, 32, 1600, 2), (1, 33, 1600, 6),
+                                           (2, 131, 1900, 6), (1, 300, 2900, 6)])
+def test_flash_attention_four_wave_rule_with_gate_and_split(b, t, l, variant):
+    """20 query / 5 K/V heads at lengths where the automatic choice is a four-wave form with 64-key
+    tiles (variant 2 up to 1632 tokens on 256 CUs, 6 beyond), as the blocks call it: gate fused, text
+    and image rows split inside a tile, ragged lengths, one and two items. The automatic choice is the
+    forced variant bit for bit, and both are held against the oracle."""
+    h, hkv, n = 20, 5, t + l
+    q, k, v, qd, kd, vt = _attn_inputs(b, h, hkv, n, 24)
+    gate = torch.randn(b, n, h * 128, generator=gen(25)).to(torch.bfloat16)
+    gy, gx = (a.reshape(-1, h * 128).contiguous().to(DEV) for a in (gate[:, :t], gate[:, t:]))
+    outs = []
+    for forced in (-1, variant):
+        oy, ox = (torch.zeros_like(a) for a in (gy, gx))
+        _lib.call("iris_flash_attn_force_variant", forced)
+        try:
+            K.flash_attention(qd, kd, vt, n, oy, ox, n_split=t, gate0=gy, gate1=gx)
+        finally:
+            _lib.call("iris_flash_attn_force_variant", -1)
+        outs.append(torch.cat([oy.view(b, t, h, 128), ox.view(b, l, h, 128)], 1).float().cpu())
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert torch.equal(*outs)
+    sel = torch.cat([torch.arange(0, n, 5), torch.arange(max(0, t - 40), t + 40), torch.arange(n - 40, n)])
+    for i in range(b):
+        for hh in (0, 3, 7, 19):
+            plain = O.attention(q[i:i + 1, hh:hh + 1, sel].float(), k[i:i + 1, hh // 4:hh // 4 + 1].float(),
+                                v[i:i + 1, hh // 4:hh // 4 + 1].float())[0, 0]
+            gates = torch.sigmoid(gate[i, sel, hh * 128:(hh + 1) * 128].float())
+            for got in outs:
+                close_attention(got[i, sel, hh], plain * gates)
+                close_attention(got[i, sel, hh] / gates, plain)
 
 
 # -- attention at the magnitudes of the trained model -----------------------------------------

@@ -158,11 +158,51 @@ def test_qk_store_of_whole_items_beside_an_empty_ragged_group():
     assert torch.all(out[:, :512] == 5.0) and torch.equal(out[:, 512:], plain[:, 512:])
 
 
+@pytest.mark.parametrize("tokens,batch", [((4096, 300), 1), ((1500,), 2), ((2000, 77), 1)])
+def test_paired_qkv_store_of_ragged_items(tokens, batch):
+    """q | k | v | gate of 20 query and 5 K/V heads at ragged row counts that the automatic choice runs
+    as the 256 x 256 store paired with 288 x 160 gate columns (on 256 CUs), the V heads through the
+    output: exactly the plain product and qkv_prepare."""
+    g = torch.Generator(device=DEV).manual_seed(46)
+    heads, kv_heads, k = 20, 5, 2560
+    n, v_col, n_qkv = 50 * 128, 25 * 128, 30 * 128
+    offsets = [tokens[1], 0] if len(tokens) == 2 else [0]
+    n_pad = (sum(tokens) + 63) // 64 * 64
+    cos, sin = (torch.randn(n_pad, 64, generator=g, device=DEV) for _ in range(2))
+    xs, ws = [randn(g, batch * t, k) for t in tokens], [randn(g, n, k, scale=0.02) for _ in tokens]
+    gains = [[1 + 0.1 * torch.randn(128, generator=g, device=DEV) for _ in tokens] for _ in range(2)]
+    bufs = [[torch.full((batch, h, *s), 3.0, device=DEV, dtype=torch.bfloat16)
+             for h, s in ((heads, (n_pad, 128)), (kv_heads, (n_pad, 128)), (kv_heads, (128, n_pad)))] for _ in range(2)]
+    plain = [forced(15, lambda x=x, w=w: K.linear(x, w)) for x, w in zip(xs, ws)]
+    for out, qw, kw, t, off in zip(plain, *gains, tokens, offsets):
+        K.qkv_prepare(out.view(batch, t, n), qw, kw, cos, sin, 1e-6, heads, kv_heads, *bufs[0], 0, heads * 128, v_col,
+                      off)
+    outs = [torch.full((batch * t, n), 5.0, device=DEV, dtype=torch.bfloat16) for t in tokens]
+    K.linear_qk_rope(xs, ws, outs, *gains, cos, sin, 1e-6, heads, kv_heads, *bufs[1][:2], list(tokens), offsets,
+                     vt=bufs[1][2], any_rows=True)
+    for got, want in zip(bufs[1], bufs[0]):
+        assert torch.equal(got, want)
+    for out, ref in zip(outs, plain):
+        assert torch.equal(out[:, n_qkv:], ref[:, n_qkv:]) and torch.all(out[:, :v_col] == 5.0)
+
+
 def test_ring_refuses_a_k_loop_shorter_than_its_ring():
     x, w = torch.zeros(8, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(64, 128, device=DEV, dtype=torch.bfloat16)
     with pytest.raises(Exception, match="ring"):
         forced(19, lambda: K.linear(x, w))
     assert torch.all(K.linear(x, w) == 0)  # the automatic choice takes another tile
+
+
+@pytest.mark.parametrize("k", [64, 128, 192])
+@pytest.mark.parametrize("m", [1, 77, 333])
+def test_automatic_choice_for_k_loops_around_the_smallest_ring(k, m):
+    """One and two K tiles fit no ring, three the smallest one only."""
+    g = torch.Generator(device=DEV).manual_seed(47)
+    x, w = randn(g, m, k), randn(g, 448, k, scale=0.1)
+    for kwargs in ({}, {"out_dtype": torch.float32}, {"swiglu": True}):
+        assert torch.equal(K.linear(x, w, **kwargs), forced(16, lambda: K.linear(x, w, **kwargs)))
+    prod = x.double() @ w.double().T  # k <= 192 products of N(0, 0.1): FP32 sums within 1e-5
+    torch.testing.assert_close(K.linear(x, w, out_dtype=torch.float32).double(), prod, rtol=1e-5, atol=1e-5)
 
 
 @pytest.mark.parametrize("n,k,swiglu", [(2560, 2560, False), (13696, 2560, True), (2560, 6848, False)])
