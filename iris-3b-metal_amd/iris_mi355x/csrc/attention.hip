@@ -803,7 +803,10 @@ extern "C" int iris_flash_attn(const void* q, const void* k, const void* vt, int
   // registers (variant 1). One item, us, variant 1 / 2 / 6 / 5: 154 tokens 11.0 / 11.0 / 11.5 /
   // 21, 333: 14.9 / 14.0 / 15.1 / 28, 1280: 34.8 / 29.5 / 31.6 / 57, 1632: 43 / 38 / 39 / 69, 2560:
   // 87 / 76 / 74 / 99, 3200: 115 / 105 / 99 / 121, 4096: 217 / 195 / 192 / 162; two items at 2560:
-  // 167 / 150 / 145 / 208. One query head per K/V head (the pixel stage): variant 2.
+  // 167 / 150 / 145 / 208, at 333 16.4 / 15.5 / 16.5 / 28, 1000: 41 / 38 / 39 / 53, 1632: 65 / 64 / 61 / 73;
+  // four at 333 19.0 / 18.6 / 19.9 / 32, 640: 33.0 / 31.6 / 31.3 / 41, 1280: 96 / 90 / 88 / 125. Where a
+  // batch's workgroups fit three per CU (variant 1) but not two, variant 1 is up to 5% ahead (four items at
+  // 1000: 72 / 76 / 74 / 58). One query head per K/V head (the pixel stage): variant 2.
   // The choice depends on one batch item's shape only: variant 5 rounds differently from
   // variant 1, and a row's result must not depend on the other items of its batch.
   int variant = g_attn_variant;

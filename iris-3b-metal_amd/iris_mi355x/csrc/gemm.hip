@@ -15,7 +15,7 @@
 //   two of its GEMMs in one grid (SwiGLU's two column parts; the q|k|v store and the gate
 //   columns beside it), which saves the boundary between two launches.
 // - gemm_ring_kernel (few rows): four waves on the same MFMA, small tiles (32 x 64 .. 192 x 128) with
-//   K tiles global -> LDS by buffer_load_dwordx4 ... lds, three to eight of them in flight.
+//   K tiles global -> LDS by buffer_load_dwordx4 ... lds into a ring of three to eight of them.
 // - gemm_w4_kernel: gemm_w4h_kernel's design on v_mfma_f32_32x32x16_bf16 (256 x 256, 192 x 256),
 //   forced-only (a tuning and test reference).
 // - gemm_kernel: eight waves, K tiles global -> LDS with buffer_load_dwordx4 ... lds into a ring
@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(256) void gemm_w4h_pair_kernel(GemmArgs p1, GemmArg
 // it into LDS (128 x 128, 107 K tiles: 31 us for the loads alone, 29 for the MFMAs alone, 50 to 57
 // for all), so small tiles that put the call on every CU are worth their extra traffic. A weight
 // read from HBM takes ~2000 clocks, a K tile 128 .. 512 of MFMAs: the ring keeps STAGES - 1 K
-// tiles (72 .. 140 KB per CU) in flight with no registers, where the register-staged kernels
+// tiles (80 .. 120 KB per CU) in flight with no registers, where the register-staged kernels
 // above hold two. Measured (2560 columns, K = 6848, weights from HBM): 333 rows 62 -> 24 us, 64
 // rows 59 -> 22 us, 924 rows 62 -> 49 us; SwiGLU 333 x 13696 x 2560 45 -> 34 us; q|k|v|gate of a
 // 256 x 256 image with 77 text tokens 109 -> 24 us. Each output sums k in the order of
@@ -1696,7 +1696,7 @@ bool mfma16_family(int epilogue) { return epilogue == IRIS_EPI_NONE || epilogue 
 
 bool allowed(const Candidate& c, int epilogue) {
   const TileShape t = kTiles[c.tile];
-  return t.mfma16() == mfma16_family(epilogue) && !(epilogue == IRIS_EPI_SILU_MUL && !t.swiglu()) &&
+  return t.w4h == mfma16_family(epilogue) && !(epilogue == IRIS_EPI_SILU_MUL && !t.swiglu()) &&
          !(epilogue == IRIS_EPI_SILU && (t.w4 || t.w4h));
 }
 
@@ -1753,8 +1753,10 @@ SplitPlan plan_split(const int* m, int groups, int n, int epilogue, int forced) 
 // box over 40 and 107 K tiles (2560 columns, K = 2560 and 6848, weights from HBM) at the row counts
 // that fill one round. The larger tiles do more work per byte they stage, the smaller ones leave
 // fewer CUs idle: 64 x 64 runs 333 x 2560 x 6848 in 24 us (240 tiles) where 128 x 160 took 62 (48
-// tiles), 96 x 128 runs q|k|v|gate of 333 rows in 24 us; from ~1300 rows on the four-wave tiles
-// fill the chip and their larger wave blocks win (1848 x 2560 x 2560: 30 us against 31).
+// tiles), 96 x 128 runs q|k|v|gate of 333 rows in 24 us. At 2560 columns the plan takes them up to 1536
+// rows (1848 x 2560 x 2560: level at 31 us) and 192 x 128 again from 2049 to 2304, where they fill one round
+// and the four-wave tiles none (2304 x 2560 x 2560 36 us against 46, K = 6848 80 against 107); q|k|v|gate of
+// 6400 columns up to 1280 rows, SwiGLU of 13696 up to 384.
 struct RingTile {
   int tile;
   double ktile_us, fixed_us;
@@ -1763,7 +1765,9 @@ constexpr RingTile kRingTiles[] = {{18, 0.158, 5.5}, {19, 0.166, 6.4}, {20, 0.21
                                    {23, 0.290, 9.5}, {24, 0.345, 10.0}, {25, 0.450, 9.5}, {26, 0.545, 9.5}};
 // Ring launches of several rounds run further above the model inside a forward than the four-wave ones
 // (SwiGLU of 256 + 77 rows, 428 tiles of 96 x 128 in two rounds: 44 us alone, 56 in the forward, where
-// 162 tiles of 192 x 256 in one take 49), so they must win by as much.
+// 162 tiles of 192 x 256 in one take 49), so they must win by as much. Alone, no launch of 1 to 8704 rows
+// that this takes to ring tiles ran slower than on the four-wave plan (K = 256 to 6848, 640 to 16384 columns,
+// one and two groups).
 constexpr double kRingRounds = 1.1;
 // The four-wave tiles in the same terms: tile area / (rate x this) per K tile, a first round's and a
 // further round's extra (the next tile's loads overlap a persistent round's output), and what the
@@ -2075,17 +2079,17 @@ extern "C" int iris_gemm_bf16_grouped(int groups, const void* const* a, const vo
 }
 
 static int qk_rope_gemm(bool any_rows, int groups, const void* const* a, const void* const* b, void* const* c,
-                                      const int* m, int n, int k, long lda, long ldb, long ldc,
-                                      const float* const* q_weight, const float* const* k_weight,
-                                      const int* rows_per_batch, const int* dst_offset, const float* cos_table,
-                                      const float* sin_table, long table_rows, void* q, void* k_out, int heads,
-                                      int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream) {
+                        const int* m, int n, int k, long lda, long ldb, long ldc, const float* const* q_weight,
+                        const float* const* k_weight, const int* rows_per_batch, const int* dst_offset,
+                        const float* cos_table, const float* sin_table, long table_rows, void* q, void* k_out, int heads,
+                        int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream) {
   IRIS_REQUIRE(groups == 1 || groups == 2, "gemm_qk_rope: 1 or 2 groups");
   IRIS_REQUIRE(heads > 0 && kv_heads > 0 && n % 128 == 0 && n >= (heads + kv_heads) * 128,
                "gemm_qk_rope: n (%d) must be whole 128-wide heads covering the %d Q and %d K heads", n, heads,
                kv_heads);
   IRIS_REQUIRE(k > 0 && k % kBK == 0, "gemm_qk_rope: need k > 0 and k %% 64 == 0 (got %d)", k);
-  IRIS_REQUIRE(lda >= k && ldb >= k && lda % 8 == 0 && ldb % 8 == 0, "gemm_qk_rope: lda/ldb must be >= k and multiples of 8");
+  IRIS_REQUIRE(lda >= k && ldb >= k && lda % 8 == 0 && ldb % 8 == 0,
+               "gemm_qk_rope: lda/ldb must be >= k and multiples of 8");
   IRIS_REQUIRE(ldc >= n && ldc % 8 == 0, "gemm_qk_rope: ldc must be >= n and a multiple of 8");
   IRIS_REQUIRE(q && k_out && cos_table && sin_table && q_weight && k_weight && rows_per_batch && dst_offset,
                "gemm_qk_rope: null pointer");
@@ -2174,35 +2178,31 @@ static int qk_rope_gemm(bool any_rows, int groups, const void* const* a, const v
   bool whole = true;
   for (int i = 0; i < groups; ++i)
     whole = whole && (m[i] == 0 || (rows_per_batch[i] % 256 == 0 && dst_offset[i] % 16 == 0));
-  if (vt && !whole) {
-    const int rc = qk_rope_gemm(false, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch,
-                                dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, nullptr,
-                                0, eps, stream);
+  if (!whole) qk.vt = nullptr;
+  int rc;
+  if (n <= n_qkv) {
+    rc = gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, kQkRopeTile, stream, &qk);
+  } else {
+    // the columns after the V heads (the gate columns of a q | k | v | gate weight) are a plain
+    // product into c beside the store, in the same launch where a pair kernel exists
+    GemmArgs a1, a2;
+    rc = make_args(a1, groups, a, b, nullptr, c, m, n_qkv, k, lda, ldb, ldc, kEpiQkRope, kQkRopeTile, &qk);
     if (rc != IRIS_OK) return rc;
+    const void* b2[2];
+    void* c2[2];
     for (int i = 0; i < groups; ++i) {
-      const int vrc = m[i] == 0 ? IRIS_OK
-                                : iris_v_heads_t(c[i], vt, m[i] / rows_per_batch[i], rows_per_batch[i], n_vt, kv_heads,
-                                                 dst_offset[i], ldc, (heads + kv_heads) * 128L, stream);
-      if (vrc != IRIS_OK) return vrc;
+      b2[i] = b[i] ? static_cast<const bf16*>(b[i]) + static_cast<long>(n_qkv) * ldb : nullptr;
+      c2[i] = c[i] ? static_cast<bf16*>(c[i]) + n_qkv : nullptr;
     }
-    return IRIS_OK;
+    rc = make_args(a2, groups, a, b2, nullptr, c2, m, n - n_qkv, k, lda, ldb, ldc, IRIS_EPI_NONE, tile2, nullptr);
+    if (rc != IRIS_OK) return rc;
+    rc = launch_two(a1, kQkRopeTile, kEpiQkRope, a2, tile2, IRIS_EPI_NONE, IRIS_BF16, stream);
   }
-  if (n <= n_qkv)
-    return gemm_part(groups, a, b, nullptr, c, m, IRIS_BF16, n, k, lda, ldb, ldc, kEpiQkRope, kQkRopeTile, stream, &qk);
-  // the columns after the V heads (the gate columns of a q | k | v | gate weight) are a plain
-  // product into c beside the store, in the same launch where a pair kernel exists
-  GemmArgs a1, a2;
-  int rc = make_args(a1, groups, a, b, nullptr, c, m, n_qkv, k, lda, ldb, ldc, kEpiQkRope, kQkRopeTile, &qk);
-  if (rc != IRIS_OK) return rc;
-  const void* b2[2];
-  void* c2[2];
-  for (int i = 0; i < groups; ++i) {
-    b2[i] = b[i] ? static_cast<const bf16*>(b[i]) + static_cast<long>(n_qkv) * ldb : nullptr;
-    c2[i] = c[i] ? static_cast<bf16*>(c[i]) + n_qkv : nullptr;
-  }
-  rc = make_args(a2, groups, a, b2, nullptr, c2, m, n - n_qkv, k, lda, ldb, ldc, IRIS_EPI_NONE, tile2, nullptr);
-  if (rc != IRIS_OK) return rc;
-  return launch_two(a1, kQkRopeTile, kEpiQkRope, a2, tile2, IRIS_EPI_NONE, IRIS_BF16, stream);
+  for (int i = 0; rc == IRIS_OK && vt && !whole && i < groups; ++i)
+    if (m[i] > 0)
+      rc = iris_v_heads_t(c[i], vt, m[i] / rows_per_batch[i], rows_per_batch[i], n_vt, kv_heads, dst_offset[i], ldc,
+                          (heads + kv_heads) * 128L, stream);
+  return rc;
 }
 
 // (with vt, iris_gemm_bf16_qk_rope takes whole 256-row items only, iris_gemm_bf16_qkv any)
@@ -2212,17 +2212,19 @@ extern "C" int iris_gemm_bf16_qk_rope(int groups, const void* const* a, const vo
                                       const int* rows_per_batch, const int* dst_offset, const float* cos_table,
                                       const float* sin_table, long table_rows, void* q, void* k_out, int heads,
                                       int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream) {
-  return qk_rope_gemm(false, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch, dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, vt, n_vt, eps, stream);
+  return qk_rope_gemm(false, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch, dst_offset,
+                      cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, vt, n_vt, eps, stream);
 }
 
-extern "C" int iris_gemm_bf16_qkv(int groups, const void* const* a, const void* const* b, void* const* c,
-                                      const int* m, int n, int k, long lda, long ldb, long ldc,
-                                      const float* const* q_weight, const float* const* k_weight,
-                                      const int* rows_per_batch, const int* dst_offset, const float* cos_table,
-                                      const float* sin_table, long table_rows, void* q, void* k_out, int heads,
-                                      int kv_heads, long n_dst, void* vt, long n_vt, float eps, hipStream_t stream) {
+extern "C" int iris_gemm_bf16_qkv(int groups, const void* const* a, const void* const* b, void* const* c, const int* m,
+                                  int n, int k, long lda, long ldb, long ldc, const float* const* q_weight,
+                                  const float* const* k_weight, const int* rows_per_batch, const int* dst_offset,
+                                  const float* cos_table, const float* sin_table, long table_rows, void* q, void* k_out,
+                                  int heads, int kv_heads, long n_dst, void* vt, long n_vt, float eps,
+                                  hipStream_t stream) {
   IRIS_REQUIRE(vt, "gemm_qkv: null vt");
-  return qk_rope_gemm(true, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch, dst_offset, cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, vt, n_vt, eps, stream);
+  return qk_rope_gemm(true, groups, a, b, c, m, n, k, lda, ldb, ldc, q_weight, k_weight, rows_per_batch, dst_offset,
+                      cos_table, sin_table, table_rows, q, k_out, heads, kv_heads, n_dst, vt, n_vt, eps, stream);
 }
 
 extern "C" int iris_gemm_bf16(const void* a, const void* b, const float* bias, void* c, int c_dtype, int m, int n,

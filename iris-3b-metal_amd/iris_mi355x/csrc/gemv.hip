@@ -10,7 +10,8 @@
 // One launch runs the image and the text core (they share their inputs), and the first timestep
 // layer computes the sinusoidal features it reads, so the chain is three launches: 51 -> 44 us per
 // denoise step.
-// gemv_kernel: any k and batch whose inputs do not fit the registers (more than 20 chunks per lane).
+// It is instantiated for the widths in use, one or five chunks per lane: k <= 512 and 2056 <= k <= 2560.
+// gemv_kernel: every other k, and inputs that are not 16-byte aligned.
 // Both add a row's products in the same order, so they agree bit for bit.
 #include "iris_common.hpp"
 
@@ -212,13 +213,14 @@ bool launch_batch(GemvLaunch& a, int jobs, int nb, hipStream_t stream) {
   switch (nb) {
     case 1: launch_rows<NCH, 1>(a, jobs, stream); return true;
     case 2: launch_rows<NCH, 2>(a, jobs, stream); return true;
-    case 3: if constexpr (3 * NCH <= 20) { launch_rows<NCH, 3>(a, jobs, stream); return true; } break;
-    case 4: if constexpr (4 * NCH <= 20) { launch_rows<NCH, 4>(a, jobs, stream); return true; } break;
+    case 3: launch_rows<NCH, 3>(a, jobs, stream); return true;
+    case 4: launch_rows<NCH, 4>(a, jobs, stream); return true;
   }
   return false;
 }
 
-// The register form where it is instantiated (the chunks per lane of the widths in use: 256, 2560).
+// The register form where it is instantiated: one chunk per lane (timestep features, also those that
+// a launch computes itself: at most 512 wide) or five (the model's width).
 bool launch_registers(GemvLaunch& a, int jobs, int nb, hipStream_t stream) {
   if (!a.freqs && !aligned(a.x, 16)) return false;
   const int nch = (a.k / 8 + kWave - 1) / kWave;
@@ -239,7 +241,6 @@ int gemv_launch(const GemvLaunch& whole, int jobs, int batch, hipStream_t stream
       a.job[j].out += static_cast<long>(b0) * a.job[j].n;
     }
     if (!launch_registers(a, jobs, nb, stream)) {
-      if (a.freqs) return fail(IRIS_E_UNSUPPORTED, "timestep_gemv: at most 256 frequencies");
       for (int j = 0; j < jobs; ++j) {
         const GemvJob& g = a.job[j];
         const dim3 grid((g.n + kRowsPerBlock - 1) / kRowsPerBlock);

@@ -534,8 +534,9 @@ def linear_qk_rope(xs, weights, outs, q_weights, k_weights, cos: torch.Tensor, s
               f"with vt the weight must hold {heads} Q, {kv_heads} K and {kv_heads} V heads "
               f"(at least {(heads + 2 * kv_heads) * HEAD_DIM} rows), got {n}")
     L.call(
-        "iris_gemm_bf16_qkv" if any_rows and vt is not None else "iris_gemm_bf16_qk_rope", groups, L.pointer_array([L.ptr(x) for x in x2]),
-        L.pointer_array([L.ptr(w) for w in weights]), L.pointer_array([L.ptr(o) for o in o2]),
+        "iris_gemm_bf16_qkv" if any_rows and vt is not None else "iris_gemm_bf16_qk_rope", groups,
+        L.pointer_array([L.ptr(x) for x in x2]), L.pointer_array([L.ptr(w) for w in weights]),
+        L.pointer_array([L.ptr(o) for o in o2]),
         L.int_array([x.shape[0] for x in x2]), n, kdim, x2[0].stride(0), weights[0].stride(0), o2[0].stride(0),
         L.pointer_array([L.ptr(w) for w in q_weights]), L.pointer_array([L.ptr(w) for w in k_weights]),
         L.int_array(list(rows_per_batch)), L.int_array(list(offsets)), L.ptr(cos), L.ptr(sin), cos.shape[0],
